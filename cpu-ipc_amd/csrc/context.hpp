@@ -88,6 +88,7 @@ struct SolveBuffers {
     DBuf<double> G;                           // factor preconditioner at the lower BSR entries
     DBuf<float> Gf;
     DBuf<int> mirror;                         // index of the transposed entry
+    DBuf<int> big;                            // block rows with a large factor pattern, and their number
     DBuf<double> vil, Gil;                    // interleaved copies for the row products
     DBuf<float> vilf, Gilf;
     size_t ne = 0;                            // BSR entry capacity (sentinels included)

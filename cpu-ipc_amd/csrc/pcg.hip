@@ -490,122 +490,172 @@ __global__ void zero_f(int n, float* __restrict__ x) {
 // row of L^-1, L the Cholesky factor of A[P,P]: then (G A G^T)_ii = I and G minimizes the
 // Kaporin condition number over the pattern (Kolotilina & Yeremin's factorized sparse
 // approximate inverse, in 3x3 blocks).  One wavefront per block row; A[P,P] in LDS.
+//
+// A row's cost is a chain of n dependent columns (a square root and a division each), so what
+// counts is how many rows a CU has in flight and what a column costs.  M is packed by columns
+// (no upper half: n (n + 1) / 2 doubles), which makes a column's reads over the lanes
+// contiguous, and the factorisation is left-looking with lane = matrix row: two LDS reads and
+// an FMA per element, no index arithmetic, no barrier (the work-group is one wavefront).  The
+// LDS follows the row's size class: at most 10 blocks (3.7 KB; lattice interiors have 4 to 10,
+// as many rows in flight as the wavefront slots allow), then 24 (21 KB) for the rows of
+// vertices in contact, which the first launch lists for the second.  Solve set-up on
+// the system of four 20^3 cubes in contact (37,044 rows) 4.34 -> 1.51 ms, of 24 scenes of up
+// to 20^3 cells (80,390 rows) 7.96 -> 1.92 ms.
 constexpr int kFsaiMax = 24;                   // blocks per row pattern
-constexpr int kFsaiN = 3 * kFsaiMax;           // dense order
-constexpr int kFsaiLd = kFsaiN + 1;            // padded leading dimension
+constexpr int kFsaiSmall = 10;                 // blocks per row of the first launch
 
 __device__ inline int find_col(const int* __restrict__ col, int lo, int hi, int c) {
     while (lo < hi) { const int m = (lo + hi) >> 1; if (col[m] < c) lo = m + 1; else hi = m; }
     return lo;
 }
+// (r, c), r >= c, of an n x n lower triangle packed by columns
+__device__ inline int packed(int n, int c, int r) { return c * n - (c * (c - 1)) / 2 + (r - c); }
 
-__global__ __launch_bounds__(64) void fsai_rows(int V, const int* __restrict__ rowptr, const int* __restrict__ col,
-                                                const double* __restrict__ val, double* __restrict__ G) {
-    __shared__ double M[kFsaiN * kFsaiLd];
-    __shared__ double Z[kFsaiN * 3];
-    __shared__ int P[kFsaiMax], Pe[kFsaiMax];
-    __shared__ int np_sh;
-    __shared__ double red[64];
+// One row, by one wavefront.  K: the most blocks of a row; rows with more go to big (their
+// number in *nbig), K == kFsaiMax drops the smallest blocks instead.
+template <int K>
+__device__ inline void fsai_row(int i, const int* __restrict__ rowptr, const int* __restrict__ col, const double* __restrict__ val,
+                                double* __restrict__ G, double* __restrict__ M, int* __restrict__ P, int* __restrict__ Pe,
+                                int* __restrict__ big, int* __restrict__ nbig) {
     const int lane = threadIdx.x;
-    for (int i = blockIdx.x; i < V; i += gridDim.x) {
-        const int e0 = rowptr[i], e1 = rowptr[i + 1];
-        const int ediag = find_col(col, e0, e1, i);           // diagonal entry of row i (present)
-        const int nl = ediag - e0;                              // off-diagonal lower candidates
-        // choose the candidates: all, or the kFsaiMax-1 largest by Frobenius norm (ties by column)
-        for (int e = e0 + lane; e < e1; e += 64) {              // clear this row's G entries
-            for (int k = 0; k < 9; ++k) G[(size_t)9 * e + k] = 0.0;
-        }
-        __syncthreads();
-        if (lane == 0) np_sh = 0;
-        __syncthreads();
-        for (int c = lane; c < nl; c += 64) {
-            bool keep = true;
-            if (nl > kFsaiMax - 1) {
+    const int e0 = rowptr[i], e1 = rowptr[i + 1];
+    const int ediag = find_col(col, e0, e1, i);           // diagonal entry of row i (present)
+    const int nl = ediag - e0;                            // off-diagonal lower candidates
+    if (K < kFsaiMax && nl > K - 1) {
+        if (lane == 0) big[atomicAdd(nbig, 1)] = i;
+        return;
+    }
+    const bool all = nl <= K - 1;
+    const int k = all ? nl + 1 : K;
+    // the pattern's entries in column order, the diagonal last; the others' blocks are zero
+    if (all) {
+        for (int a = lane; a < k; a += 64) { Pe[a] = e0 + a; P[a] = col[e0 + a]; }
+        for (size_t t = (size_t)9 * (ediag + 1) + lane; t < (size_t)9 * e1; t += 64) G[t] = 0.0;
+    } else {
+        // the K - 1 largest by Frobenius norm (ties by column)
+        int kept = 0;
+        for (int c0 = 0; c0 < nl; c0 += 64) {
+            const int c = c0 + lane;
+            bool keep = false;
+            if (c < nl) {
                 double nc = 0;
-                for (int k = 0; k < 9; ++k) nc += val[(size_t)9 * (e0 + c) * 1 + k] * val[(size_t)9 * (e0 + c) + k];
+                for (int q = 0; q < 9; ++q) nc += val[(size_t)9 * (e0 + c) + q] * val[(size_t)9 * (e0 + c) + q];
                 int rank = 0;
                 for (int o = 0; o < nl; ++o) {
                     double no = 0;
-                    for (int k = 0; k < 9; ++k) no += val[(size_t)9 * (e0 + o) + k] * val[(size_t)9 * (e0 + o) + k];
+                    for (int q = 0; q < 9; ++q) no += val[(size_t)9 * (e0 + o) + q] * val[(size_t)9 * (e0 + o) + q];
                     rank += (no > nc) || (no == nc && o < c);
                 }
-                keep = rank < kFsaiMax - 1;
+                keep = rank < K - 1;
             }
+            const unsigned long long m = __ballot(keep);
             if (keep) {
-                const int slot = atomicAdd(&np_sh, 1);
+                const int slot = kept + __popcll(m & ((1ull << lane) - 1));
                 Pe[slot] = e0 + c;
+                P[slot] = col[e0 + c];
             }
+            kept += __popcll(m);
         }
-        __syncthreads();
-        const int k = np_sh + 1;
-        if (lane == 0) {
-            // sort the kept entries by column (insertion sort, k <= kFsaiMax), diagonal last
-            for (int a = 1; a < k - 1; ++a) {
-                const int v = Pe[a];
-                int b = a - 1;
-                while (b >= 0 && Pe[b] > v) { Pe[b + 1] = Pe[b]; --b; }
-                Pe[b + 1] = v;
-            }
-            Pe[k - 1] = ediag;
-            for (int a = 0; a < k; ++a) P[a] = col[Pe[a]];
-        }
-        __syncthreads();
-        const int n = 3 * k;
-        // M = A[P,P] (lower blocks looked up in the block rows of P; upper by symmetry)
-        for (int ab = lane; ab < k * k; ab += 64) {
-            const int a = ab / k, b = ab % k;
-            if (b > a) continue;
-            const int ra = P[a];
-            const int rs = rowptr[ra], re = rowptr[ra + 1];
-            const int f = find_col(col, rs, re, P[b]);
-            const bool has = f < re && col[f] == P[b];
-            for (int u = 0; u < 3; ++u)
-                for (int v = 0; v < 3; ++v) {
-                    const double m = has ? val[(size_t)9 * f + 3 * u + v] : 0.0;   // A_{P_a P_b}(u, v)
-                    M[(3 * a + u) * kFsaiLd + 3 * b + v] = m;
-                    M[(3 * b + v) * kFsaiLd + 3 * a + u] = m;
+        if (lane == 0) { Pe[K - 1] = ediag; P[K - 1] = i; }
+        for (size_t t = (size_t)9 * e0 + lane; t < (size_t)9 * e1; t += 64) G[t] = 0.0;
+    }
+    __syncthreads();
+    const int n = 3 * k;
+    // M = A[P,P], lower triangle: blocks (a, b <= a) looked up in the block rows of P
+    for (int ab = lane; ab < k * (k + 1) / 2; ab += 64) {
+        int a = (int)((sqrtf(8.0f * (float)ab + 1.0f) - 1.0f) * 0.5f);
+        while ((a + 1) * (a + 2) / 2 <= ab) ++a;
+        while (a * (a + 1) / 2 > ab) --a;
+        const int b = ab - a * (a + 1) / 2;
+        const int rs = rowptr[P[a]], re = rowptr[P[a] + 1];
+        const int f = find_col(col, rs, re, P[b]);
+        const bool has = f < re && col[f] == P[b];
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+#pragma unroll
+            for (int v = 0; v < 3; ++v)
+                if (a != b || u >= v) M[packed(n, 3 * b + v, 3 * a + u)] = has ? val[(size_t)9 * f + 3 * u + v] : 0.0;   // A_{P_a P_b}(u, v)
+    }
+    __syncthreads();
+    // Cholesky M = L L^T, left-looking: lane r holds row r (and row 64 + r when 3 K > 64)
+    constexpr int R = (3 * K + 63) / 64;
+    for (int c = 0; c < n; ++c) {
+        double s[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const int r = lane + 64 * q;
+            double s0 = 0.0, s1 = 0.0;
+            if (r >= c && r < n) {
+                s0 = M[packed(n, c, r)];
+                int m = 0;
+                for (; m + 1 < c; m += 2) {
+                    const int b0 = packed(n, m, 0), b1 = packed(n, m + 1, 0);
+                    s0 -= M[b0 + r] * M[b0 + c];
+                    s1 -= M[b1 + r] * M[b1 + c];
                 }
-        }
-        __syncthreads();
-        // Cholesky M = L L^T in place (lower triangle)
-        for (int c = 0; c < n; ++c) {
-            if (lane == 0) M[c * kFsaiLd + c] = sqrt(fmax(M[c * kFsaiLd + c], 1e-300));
-            __syncthreads();
-            const double dc = M[c * kFsaiLd + c];
-            for (int r = c + 1 + lane; r < n; r += 64) M[r * kFsaiLd + c] /= dc;
-            __syncthreads();
-            const int m = n - c - 1;
-            for (int idx = lane; idx < m * m; idx += 64) {
-                const int r = c + 1 + idx / m, q = c + 1 + idx % m;
-                if (q <= r) M[r * kFsaiLd + q] -= M[r * kFsaiLd + c] * M[q * kFsaiLd + c];
+                if (m < c) { const int b0 = packed(n, m, 0); s0 -= M[b0 + r] * M[b0 + c]; }
             }
-            __syncthreads();
+            s[q] = s0 + s1;
         }
-        // L^T Z = E (last three unit columns), bottom-up; lanes split the dot products
-        for (int r = n - 1; r >= 0; --r) {
-            for (int qq = 0; qq < 3; ++qq) {
-                double acc = 0.0;
-                for (int s2 = r + 1 + lane; s2 < n; s2 += 64) acc += M[s2 * kFsaiLd + r] * Z[s2 * 3 + qq];
-                red[lane] = acc;
-                __syncthreads();
-                for (int w = 32; w > 0; w >>= 1) {
-                    if (lane < w) red[lane] += red[lane + w];
-                    __syncthreads();
-                }
-                if (lane == 0) {
-                    const double rhs = (r == n - 3 + qq) ? 1.0 : 0.0;
-                    Z[r * 3 + qq] = (rhs - red[0]) / M[r * kFsaiLd + r];
-                }
-                __syncthreads();
-            }
-        }
-        // G_{i, P_a} (row u, column v) = Z[3a + v][u]
-        for (int idx = lane; idx < 9 * k; idx += 64) {
-            const int a = idx / 9, u = (idx % 9) / 3, v = idx % 3;
-            G[(size_t)9 * Pe[a] + 3 * u + v] = Z[(3 * a + v) * 3 + u];
+        const double piv = R > 1 && c >= 64 ? __shfl(s[R - 1], c - 64) : __shfl(s[0], c);
+        const double d = sqrt(fmax(piv, 1e-300));
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const int r = lane + 64 * q;
+            if (r == c) M[packed(n, c, r)] = d;
+            else if (r > c && r < n) M[packed(n, c, r)] = s[q] / d;
         }
         __syncthreads();
     }
+    // L^T Z = E (last three unit columns), from the last row up: lane r keeps row r of the
+    // right-hand sides and subtracts L(s, r) z_s as each z_s is known
+    double z[R][3];
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int u = 0; u < 3; ++u) z[q][u] = (lane + 64 * q == n - 3 + u) ? 1.0 : 0.0;
+    for (int sr = n - 1; sr >= 0; --sr) {
+        const double d = M[packed(n, sr, sr)];
+        double zs[3];
+#pragma unroll
+        for (int u = 0; u < 3; ++u) zs[u] = (R > 1 && sr >= 64 ? __shfl(z[R - 1][u], sr - 64) : __shfl(z[0][u], sr)) / d;
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const int r = lane + 64 * q;
+            if (r == sr) {
+#pragma unroll
+                for (int u = 0; u < 3; ++u) z[q][u] = zs[u];
+            } else if (r < sr) {
+                const double l = M[packed(n, r, sr)];
+#pragma unroll
+                for (int u = 0; u < 3; ++u) z[q][u] -= l * zs[u];
+            }
+        }
+    }
+    // G_{i, P_a} (row u, column v) = Z[3a + v][u]
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        const int r = lane + 64 * q;
+        if (r < n) {
+            double* g = G + (size_t)9 * Pe[r / 3] + r % 3;
+#pragma unroll
+            for (int u = 0; u < 3; ++u) g[3 * u] = z[q][u];
+        }
+    }
+    __syncthreads();   // the LDS is the next row's
+}
+// rows = null: the rows [0, V) of at most K blocks, the others listed; else the listed rows
+template <int K>
+__global__ __launch_bounds__(64) void fsai_rows(int V, const int* __restrict__ rows, int* __restrict__ nrows, const int* __restrict__ rowptr,
+                                                const int* __restrict__ col, const double* __restrict__ val, double* __restrict__ G,
+                                                int* __restrict__ big) {
+    __shared__ double M[3 * K * (3 * K + 1) / 2];
+    __shared__ int P[K], Pe[K];
+    const int n = rows ? *nrows : V;
+    for (int t = blockIdx.x; t < n; t += gridDim.x) fsai_row<K>(rows ? rows[t] : t, rowptr, col, val, G, M, P, Pe, big, nrows);
+}
+__global__ void zero_one(int* __restrict__ p) {
+    if (threadIdx.x == 0) *p = 0;
 }
 // mirror[e] = index of the entry (col(e), row(e))
 __global__ void bsr_mirror(int V, const int* __restrict__ rowptr, const int* __restrict__ col, int* __restrict__ mirror) {
@@ -786,8 +836,13 @@ void build_fsai(Context& c, bool fp32) {
     w.G.resize(9 * ne);
     w.mirror.resize(ne);
     hipLaunchKernelGGL(bsr_mirror, dim3(blocks_for(V, 256)), dim3(256), 0, c.stream, V, w.rowptr.p, w.col.p, w.mirror.p);
-    const int grid = std::min(V, 256 * 16);
-    hipLaunchKernelGGL(fsai_rows, dim3(grid), dim3(64), 0, c.stream, V, w.rowptr.p, w.col.p, w.val.p, w.G.p);
+    w.big.resize((size_t)V + 1);
+    int* nbig = w.big.p + V;
+    hipLaunchKernelGGL(zero_one, dim3(1), dim3(64), 0, c.stream, nbig);
+    hipLaunchKernelGGL(fsai_rows<kFsaiSmall>, dim3(V), dim3(64), 0, c.stream, V, (const int*)nullptr, nbig, w.rowptr.p, w.col.p, w.val.p,
+                       w.G.p, w.big.p);
+    hipLaunchKernelGGL(fsai_rows<kFsaiMax>, dim3(std::min(V, 256 * 7)), dim3(64), 0, c.stream, V, (const int*)w.big.p, nbig, w.rowptr.p,
+                       w.col.p, w.val.p, w.G.p, w.big.p);
     CIPC_CHECK_LAUNCH();
     if (fp32) {
         w.Gf.resize(9 * ne);
