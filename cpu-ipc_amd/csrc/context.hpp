@@ -80,17 +80,18 @@ struct ActiveSetScratch {
 
 // Buffers of the Newton linear solve (pcg.hip).
 struct SolveBuffers {
-    DBuf<unsigned long long> key, key_sorted;
-    DBuf<int> src, src_sorted, col, rowptr;   // full symmetric 3x3-block matrix (BSR)
-    DBuf<double> val, minv;                   // FP64 blocks and block-Jacobi inverses
-    DBuf<float> valf, minvf, xf;              // FP32 copies for the mixed form
+    // full symmetric 3x3-block matrix (BSR): row starts, diagonal positions, columns, index of
+    // the transposed entry; the lower entries' counts, starts and merged blocks per row
+    DBuf<int> rowptr, dpos, col, mirror, lowcnt, lowstart, low;
+    DBuf<double> vil;                         // blocks interleaved for the products
+    DBuf<float> vilf;                         // FP32 copy for the mixed form
+    DBuf<double> val;                         // plain blocks (learned factor)
+    DBuf<double> minv;                        // block-Jacobi inverses
+    DBuf<float> minvf, xf;
     DBuf<double> r, z, p, q, x, res, part, scal, t;
-    DBuf<double> G;                           // factor preconditioner at the lower BSR entries
-    DBuf<float> Gf;
-    DBuf<int> mirror;                         // index of the transposed entry
+    DBuf<double> G, F;                        // factor at the lower entries; both its products' blocks, interleaved
+    DBuf<float> Gf, Ff;
     DBuf<int> big;                            // block rows with a large factor pattern, and their number
-    DBuf<double> vil, Gil;                    // interleaved copies for the row products
-    DBuf<float> vilf, Gilf;
     size_t ne = 0;                            // BSR entry capacity (sentinels included)
     int factor = 0;                           // factor in G: 0 none, 1 block FSAI, 2 learned
     // batch: work-group tables of the row kernels (per vertex partition) and per-scene controls
@@ -305,8 +306,6 @@ void upload_counts(Context& c);
 // Contact-record capacity for the next assembly (at least the settled contact count).
 void size_contact_records(Context& c);
 void sort_u64(Context& c, const unsigned long long* in, unsigned long long* out, int n, int bits);
-void sort_u64_pairs(Context& c, const unsigned long long* kin, unsigned long long* kout,
-                    const int* vin, int* vout, int n, int bits);
 void sort_i32_pairs(Context& c, const int* kin, int* kout, const int* vin, int* vout, int n, int bits);
 void sort_u32_pairs(Context& c, const unsigned* kin, unsigned* kout, const int* vin, int* vout, int n, int bits);
 void sort_u32_pairs(const unsigned* kin, unsigned* kout, const int* vin, int* vout, int n, int bits, hipStream_t st,
@@ -393,7 +392,7 @@ __device__ inline void energy_block_sum(double v, double* part) {
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 void friction_update(Context& c, double kappa);
-void build_solve_matrix(Context& c, bool fp32);
+void build_solve_matrix(Context& c, bool fp32, bool plain);
 // preconditioner: 0 block-Jacobi, 1 block FSAI, 2 learned factor
 // preconditioner kDirectSolve: the dense Cholesky direct solve (precision ignored)
 constexpr int kDirectSolve = 3;
@@ -401,7 +400,7 @@ constexpr int kDirectMaxDofs = 60000;   // 28.8 GB of dense factor at the limit
 void linear_solve(Context& c, int precision, int preconditioner, double rel_tol, int max_iter, SolveResult& res);
 void direct_solve(Context& c, SolveResult& res);
 void destroy_direct(Context& c);
-void build_fsai(Context& c, bool fp32);
+void build_fsai(Context& c);
 void build_learned(Context& c, bool fp32);
 void learned_set_weights(Context& c, const float* w, int64_t n);
 int64_t learned_param_count();

@@ -193,16 +193,6 @@ __global__ void fill_neg(int n, int* __restrict__ p) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = -1;
 }
-__device__ inline int find_col_g(const int* __restrict__ col, int lo, int hi, int c) {
-    while (lo < hi) { const int m = (lo + hi) >> 1; if (col[m] < c) lo = m + 1; else hi = m; }
-    return lo;
-}
-__global__ void bsr_mirror_kernel(int V, const int* __restrict__ rowptr, const int* __restrict__ col, int* __restrict__ mirror) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= V) return;
-    for (int e = rowptr[a]; e < rowptr[a + 1]; ++e) mirror[e] = find_col_g(col, rowptr[col[e]], rowptr[col[e] + 1], a);
-}
-// flags[e] = entry e is a lower off-diagonal entry; flags[ne] = 0
 __global__ void lower_flags(int ne, const int* __restrict__ row, const int* __restrict__ col, int* __restrict__ flags) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e > ne) return;
@@ -667,8 +657,6 @@ void prepare(Context& c) {
     // entries past the used ones keep row -1
     hipLaunchKernelGGL(fill_neg, dim3(blocks_for(ne, 256)), dim3(256), 0, c.stream, ne, S.row.p);
     hipLaunchKernelGGL(entry_rows, dim3(blocks_for(V, 256)), dim3(256), 0, c.stream, V, w.rowptr.p, w.col.p, S.row.p, S.diag.p);
-    w.mirror.resize(ne);
-    hipLaunchKernelGGL(bsr_mirror_kernel, dim3(blocks_for(V, 256)), dim3(256), 0, c.stream, V, w.rowptr.p, w.col.p, w.mirror.p);
     CIPC_CHECK_LAUNCH();
     // lower off-diagonal entry list (in entry order) and each entry's position in it
     S.lowpos.resize(ne + 1);
@@ -785,14 +773,14 @@ double learned_loss_grad(Context& c, const float* params, const float* host_prob
     const Layout& Y = S.lay;
     const int np = (int)Y.total;
     upload_weights(c, params);
-    build_solve_matrix(c, false);
+    build_solve_matrix(c, false, true);
     prepare(c);
     forward(c);
     SolveBuffers& w = c.solve;
     const int V = c.sc.V, ne = (int)w.ne, nl = S.nlow, n3 = 3 * V;
     // ---- loss and dG^ ----
     if (objective == 1) {
-        build_fsai(c, false);
+        build_fsai(c);
         S.dG.resize((size_t)9 * ne);
         const int nb = (int)blocks_for(ne, 256);
         S.lpart.resize(nb);

@@ -19,14 +19,6 @@ namespace cipc {
 
 constexpr unsigned long long kNoKey = ~0ull;
 
-void sort_u64_pairs(Context& c, const unsigned long long* kin, unsigned long long* kout, const int* vin, int* vout,
-                    int n, int bits) {
-    if (n <= 0) return;
-    size_t bytes = 0;
-    CIPC_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, kin, kout, vin, vout, n, 0, bits, c.stream));
-    c.tmp.reserve(bytes);
-    CIPC_HIP(hipcub::DeviceRadixSort::SortPairs(c.tmp.p, bytes, kin, kout, vin, vout, n, 0, bits, c.stream));
-}
 void sort_u64(Context& c, const unsigned long long* kin, unsigned long long* kout, int n, int bits) {
     if (n <= 0) return;
     size_t bytes = 0;

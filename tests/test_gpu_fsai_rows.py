@@ -46,6 +46,8 @@ def test_factor_rows(n):
         want = F.block_fsai(B.indptr, B.indices, np.asarray(B.data)).tocsr()
         g.solve(precision=0, rel_tol=1e-6, preconditioner=1)
         got = g.solve_factor().tocsr()
+        # the matrix's block pattern, rows in order: every lower entry found at its row
+        assert np.array_equal(got.indptr, B.tocsr().indptr) and np.array_equal(got.indices, B.tocsr().indices)
         assert np.count_nonzero(got[3 * n].toarray()) > 0
         D = (got - want).tocoo()
         top = np.asarray(abs(want).max(axis=1).todense()).ravel().reshape(-1, 3).max(axis=1).repeat(3)
