@@ -88,9 +88,11 @@ struct SolveBuffers {
     DBuf<double> val;                         // plain blocks (learned factor)
     DBuf<double> minv;                        // block-Jacobi inverses
     DBuf<float> minvf, xf;
-    DBuf<double> r, z, p, q, x, res, part, scal, t;
+    DBuf<double> r, x, res, part, scal;
     DBuf<double> G, F;                        // factor at the lower entries; both its products' blocks, interleaved
     DBuf<float> Gf, Ff;
+    DBuf<double> zp, rq, t, sums;             // vectors as the products gather them (pcg_product); per-scene sums
+    DBuf<int> active;                         // scenes not yet done
     DBuf<int> big;                            // block rows with a large factor pattern, and their number
     size_t ne = 0;                            // BSR entry capacity (sentinels included)
     int factor = 0;                           // factor in G: 0 none, 1 block FSAI, 2 learned
@@ -230,6 +232,7 @@ struct Context {
     PinnedBuf<unsigned char> pin_rb;   // staging of read_back
     PinnedBuf<unsigned long long> pin_slots;
     PinnedBuf<double> pin_energy;
+    PinnedBuf<int> pin_pcg;            // a solve's progress, written by its kernels
     bool assembled = false;    // a system exists for the linear solve
     SolveBuffers solve;
     int collisions = 0;

@@ -15,11 +15,13 @@
 // M^-1 = G^T G, either the block FSAI of the matrix or the learned factor (learned.hip).
 //
 // Scalars (alpha, beta, norms) stay on the device and are combined from per-work-group
-// partials in a fixed order (deterministic).  kCheck iterations are captured once into a
-// HIP graph and replayed; the host checks convergence after each replay and kernels
-// launched past convergence return at once.
+// partials in a fixed order (deterministic).  An iteration is one launch per true dependency
+// (pcg_product, pcg_update, pcg_factor); the host enqueues a few iterations ahead of the
+// iteration number that the device reports through pinned memory, and launches that follow
+// convergence return at once.
 #include <rocsolver/rocsolver.h>
 #include "context.hpp"
+#include "lbvh.hpp"
 
 #include <cmath>
 #include <cstring>
@@ -27,7 +29,8 @@
 namespace cipc {
 
 constexpr int kPB = 256;       // threads per work-group (one vertex = 3 DOFs per thread)
-constexpr int kCheck = 16;     // iterations between host convergence checks
+constexpr int kAhead = 6;      // iterations enqueued ahead of the device
+constexpr int kOwnSums = 2048; // partials that every work-group adds up itself (pcg_sums otherwise)
 constexpr int kMaxRefine = 64; // FP64 refinement steps of the mixed form
 
 // device scalars of one solve
@@ -36,8 +39,6 @@ struct PcgScalars {
     double rr;        // r . r
     double bn;        // ||b||
     double tol;       // absolute residual target
-    double pq;        // p . q of the current iteration
-    double beta;      // r.z' / r.z of the current iteration
     int done;         // converged (or broken down)
     int iters;
 };
@@ -76,12 +77,37 @@ __global__ void bsr_place(int nm, int V, const int* __restrict__ mrow, const int
     const int a = mrow[k];
     if (a != mcol[k]) low[lowstart[a] + atomicSub(cnt + a, 1) - 1] = k;
 }
-// Interleaved layout of the blocks for the products: entries in groups of kGL, each group
-// stored component-major (entry e, component k at (e / kGL) 9 kGL + k kGL + e % kGL), so that
-// the kGL lanes of a row, which read consecutive entries, load each component with one
-// contiguous access instead of nine 72-byte-strided ones.
+// Interleaved layout of the blocks for the products: entries in groups of kGL, a group's
+// components 0..7 in 16-byte pieces (two doubles or four floats of one entry), piece by piece
+// over the entries, then its components 8.  The kGL lanes of a row read consecutive entries, so
+// each piece is one contiguous 128-byte access: five loads a block in FP64 and three in FP32,
+// where component-major order took nine and 72-byte blocks nine strided ones.
 constexpr int kGL = 8;         // lanes per block row of a product
-__host__ __device__ inline size_t il_index(size_t e, int k) { return (e / kGL) * (9 * kGL) + (size_t)k * kGL + e % kGL; }
+template <typename T>
+struct Wide;
+template <>
+struct Wide<double> { typedef double type __attribute__((ext_vector_type(2))); };
+template <>
+struct Wide<float> { typedef float type __attribute__((ext_vector_type(4))); };
+template <typename T>
+__host__ __device__ inline size_t il_index(size_t e, int k) {
+    constexpr int W = 16 / (int)sizeof(T);
+    return (e / kGL) * (9 * kGL) + (k < 8 ? (size_t)(k / W) * (kGL * W) + (e % kGL) * W + k % W : 8 * kGL + e % kGL);
+}
+// the block of entry e, B its group's start
+template <typename T>
+__device__ inline void load_block(const T* __restrict__ B, unsigned e, T f[9]) {
+    using V = typename Wide<T>::type;
+    constexpr int W = 16 / (int)sizeof(T);
+    const V* w = reinterpret_cast<const V*>(B) + e % kGL;
+#pragma unroll
+    for (int j = 0; j < 8 / W; ++j) {
+        const V t = w[j * kGL];
+#pragma unroll
+        for (int i = 0; i < W; ++i) f[j * W + i] = t[i];
+    }
+    f[8] = B[8 * kGL + e % kGL];
+}
 // Columns, mirror indices and blocks of both entries of every merged block.  A lane finds its
 // block's two positions; the wavefront then writes its 64 blocks' components in merged order
 // (coalesced reads).  vil / vilf: interleaved, val: plain 9-double blocks; null where unused.
@@ -118,12 +144,12 @@ __global__ __launch_bounds__(256) void bsr_fill(int nm, const int* __restrict__ 
         const double v = mval[(size_t)9 * k0 + t];
         const int ct = 3 * (c % 3) + c / 3;                   // (b, a) holds the transpose
         const int cu = l < 0 ? c : ct;                         // (the diagonal block as stored)
-        if (vil) vil[il_index(u, cu)] = v;
-        if (vilf) vilf[il_index(u, cu)] = (float)v;
+        if (vil) vil[il_index<double>(u, cu)] = v;
+        if (vilf) vilf[il_index<float>(u, cu)] = (float)v;
         if (val) val[(size_t)9 * u + cu] = v;
         if (l >= 0) {
-            if (vil) vil[il_index(l, c)] = v;
-            if (vilf) vilf[il_index(l, c)] = (float)v;
+            if (vil) vil[il_index<double>(l, c)] = v;
+            if (vilf) vilf[il_index<float>(l, c)] = (float)v;
             if (val) val[(size_t)9 * l + c] = v;
         }
     }
@@ -155,24 +181,42 @@ __device__ inline void block_mv(const T* __restrict__ B, const T* __restrict__ x
     y[1] = (double)B[3] * x[0] + (double)B[4] * x[1] + (double)B[5] * x[2];
     y[2] = (double)B[6] * x[0] + (double)B[7] * x[1] + (double)B[8] * x[2];
 }
+template <typename T>
+__device__ inline void transpose3(T f[9]) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+        for (int m = 0; m < u; ++m) { const T w = f[3 * u + m]; f[3 * u + m] = f[3 * m + u]; f[3 * m + u] = w; }
+}
 // Row-parallel sparse products: kGL lanes per 3x3-block row, so that the lanes of a row read
 // consecutive blocks (coalesced), combined with cross-lane shuffles.  kRows rows per work-group.
 constexpr int kRows = kPB / kGL;
+// v + v of the lane that the data-parallel-primitive control CTRL selects: the cross-lane sums
+// go through the vector pipe (a few cycles a step) instead of LDS permutes (about a hundred)
+template <int CTRL, int ROWS = 0xf>
+__device__ inline double dpp_add(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+    return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140, kDppBcast15 = 0x142, kDppBcast31 = 0x143;
+// sum over the kGL lanes of a row, in each of them
+__device__ inline double row_sum(double v) { return dpp_add<kDppHalfMirror>(dpp_add<kDppXor2>(dpp_add<kDppXor1>(v))); }
+// sum over the wavefront, in its last lane
+__device__ inline double wave_sum(double v) {
+    return dpp_add<kDppBcast31, 0xc>(dpp_add<kDppBcast15, 0xa>(dpp_add<kDppMirror>(row_sum(v))));
+}
 template <typename T>
 __device__ inline void group_reduce3(double y[3]) {
 #pragma unroll
-    for (int o = kGL / 2; o > 0; o >>= 1) {
-        y[0] += __shfl_xor(y[0], o, kGL);
-        y[1] += __shfl_xor(y[1], o, kGL);
-        y[2] += __shfl_xor(y[2], o, kGL);
-    }
+    for (int u = 0; u < 3; ++u) y[u] = row_sum(y[u]);
 }
 template <typename T, typename X>
 __device__ inline void block_mv_il(const T* __restrict__ B, size_t e, const X* __restrict__ x, double y[3]) {
-    const T* b = B + (e / kGL) * (9 * kGL) + e % kGL;
-    y[0] = (double)b[0] * x[0] + (double)b[kGL] * x[1] + (double)b[2 * kGL] * x[2];
-    y[1] = (double)b[3 * kGL] * x[0] + (double)b[4 * kGL] * x[1] + (double)b[5 * kGL] * x[2];
-    y[2] = (double)b[6 * kGL] * x[0] + (double)b[7 * kGL] * x[1] + (double)b[8 * kGL] * x[2];
+    T f[9];
+    load_block(B + (e / kGL) * (9 * kGL), (unsigned)e, f);
+    block_mv(f, x, y);
 }
 // y = (A x)_a over entries rowptr[a] + sub, step kGL (all lanes of the group get the sum);
 // val interleaved
@@ -187,49 +231,44 @@ __device__ inline void row_product(int a, int sub, const int* __restrict__ rowpt
     }
     group_reduce3<T>(y);
 }
-// work-group sum of up to three values; thread 0 stores them at part[k * gridDim.x + blockIdx.x]
+// work-group sums of K values, the k-th stored at part[k][b]
 template <int K>
-__device__ inline void group_partials(double v[K], double* __restrict__ part) {
-    __shared__ double sh[K][kPB];
+__device__ inline void group_partials(int b, const double (&v)[K], double* const (&part)[K]) {
+    __shared__ double sh[K][kPB / 64];
 #pragma unroll
-    for (int k = 0; k < K; ++k) sh[k][threadIdx.x] = v[k];
-    __syncthreads();
-    for (int s = kPB / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s)
-#pragma unroll
-            for (int k = 0; k < K; ++k) sh[k][threadIdx.x] += sh[k][threadIdx.x + s];
-        __syncthreads();
+    for (int k = 0; k < K; ++k) {
+        const double s = wave_sum(v[k]);
+        if ((threadIdx.x & 63) == 63) sh[k][threadIdx.x >> 6] = s;
     }
-    if (threadIdx.x == 0)
+    __syncthreads();
+    if (threadIdx.x < K) {
+        double s = 0.0;
+        for (int w = 0; w < kPB / 64; ++w) s += sh[threadIdx.x][w];
 #pragma unroll
-        for (int k = 0; k < K; ++k) part[k * gridDim.x + blockIdx.x] = sh[k][0];
+        for (int k = 0; k < K; ++k)
+            if ((int)threadIdx.x == k) part[k][b] = s;
+    }
 }
-// work-group sums of two values stored to two partial arrays
-__device__ inline void group_partials2(double v[2], double* __restrict__ pa, double* __restrict__ pb) {
-    __shared__ double sh[2][kPB];
-    sh[0][threadIdx.x] = v[0];
-    sh[1][threadIdx.x] = v[1];
-    __syncthreads();
-    for (int s = kPB / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) { sh[0][threadIdx.x] += sh[0][threadIdx.x + s]; sh[1][threadIdx.x] += sh[1][threadIdx.x + s]; }
-        __syncthreads();
+// the sums of n partials of the previous kernel, in an order fixed by n, in every thread
+template <int K>
+__device__ inline void sum_partials_fixed(const double* const (&part)[K], int n, double (&out)[K]) {
+    __shared__ double sh[K][kPB / 64];
+#pragma unroll
+    for (int k = 0; k < K; ++k) out[k] = 0.0;
+    for (int i = threadIdx.x; i < n; i += kPB)
+#pragma unroll
+        for (int k = 0; k < K; ++k) out[k] += part[k][i];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const double s = wave_sum(out[k]);
+        if ((threadIdx.x & 63) == 63) sh[k][threadIdx.x >> 6] = s;
     }
-    if (threadIdx.x == 0) { pa[blockIdx.x] = sh[0][0]; pb[blockIdx.x] = sh[1][0]; }
-}
-// every work-group sums the partials of the previous kernel in the same order
-__device__ inline double sum_partials_fixed(const double* __restrict__ part, int n) {
-    __shared__ double sh[kPB];
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < n; i += kPB) acc += part[i];
-    sh[threadIdx.x] = acc;
     __syncthreads();
-    for (int s = kPB / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-        __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        out[k] = 0.0;
+        for (int w = 0; w < kPB / 64; ++w) out[k] += sh[k][w];
     }
-    const double r = sh[0];
-    __syncthreads();
-    return r;
 }
 
 // ---- work-group layout of the row kernels ----------------------------------------------
@@ -242,12 +281,17 @@ struct Layout {
     int V = 0, ng = 0;
     const int4* bl = nullptr;
     const int* gb = nullptr;
-    __device__ void block(int& scene, int& row0, int& rend) const {
+    // The work-group's place.  One system: each XCD takes a contiguous part of the rows, whose
+    // neighbours mostly lie in the same part, so that its L2 holds an eighth of the vectors
+    // and not all.  A batch stays round-robin: its scenes converge at different iterations, and
+    // contiguous parts would leave XCDs without work (13.5 us against 10.8 us a product).
+    __device__ int index() const { return bl ? (int)blockIdx.x : xcd_block(blockIdx.x, gridDim.x); }
+    __device__ void block(int b, int& scene, int& row0, int& rend) const {
         if (bl) {
-            const int4 t = bl[blockIdx.x];
+            const int4 t = bl[b];
             scene = t.x; row0 = t.y; rend = t.z;
         } else {
-            scene = 0; row0 = blockIdx.x * kRows; rend = V;
+            scene = 0; row0 = b * kRows; rend = V;
         }
     }
     __device__ void parts(int scene, int& lo, int& n) const {
@@ -265,8 +309,9 @@ __global__ __launch_bounds__(kPB) void pcg_residual(Layout L, const int* __restr
                                                     const T* __restrict__ val, const double* __restrict__ b, const T* __restrict__ x,
                                                     int x_zero, T* __restrict__ r, double* __restrict__ part_rr,
                                                     double* __restrict__ part_bb) {
+    const int wg = L.index();
     int scene, row0, rend;
-    L.block(scene, row0, rend);
+    L.block(wg, scene, row0, rend);
     const int a = row0 + threadIdx.x / kGL, sub = threadIdx.x % kGL;
     double acc[2] = {0, 0};
     if (a < rend) {
@@ -279,29 +324,7 @@ __global__ __launch_bounds__(kPB) void pcg_residual(Layout L, const int* __restr
             acc[0] = (double)(T)rv[0] * (T)rv[0] + (double)(T)rv[1] * (T)rv[1] + (double)(T)rv[2] * (T)rv[2];
         }
     }
-    group_partials2(acc, part_rr, part_bb);
-}
-// block-Jacobi: z = M^-1 r; partial of r.z; p = z when `init`
-template <typename T>
-__global__ __launch_bounds__(kPB) void prec_jacobi(Layout L, const T* __restrict__ minv, const T* __restrict__ r, T* __restrict__ z,
-                                                   T* __restrict__ p, int init, const PcgScalars* __restrict__ sc,
-                                                   double* __restrict__ part_rz) {
-    int scene, row0, rend;
-    L.block(scene, row0, rend);
-    if (sc && sc[scene].done) return;
-    const int a = row0 + threadIdx.x / kGL, sub = threadIdx.x % kGL;
-    double acc[1] = {0.0};
-    if (a < rend && sub == 0) {
-        const T rt[3] = {r[3 * a], r[3 * a + 1], r[3 * a + 2]};
-        double zv[3];
-        block_mv(minv + (size_t)9 * a, rt, zv);
-        for (int k = 0; k < 3; ++k) {
-            z[3 * a + k] = (T)zv[k];
-            if (init) p[3 * a + k] = (T)zv[k];
-        }
-        acc[0] = (double)rt[0] * (T)zv[0] + (double)rt[1] * (T)zv[1] + (double)rt[2] * (T)zv[2];
-    }
-    group_partials<1>(acc, part_rz);
+    group_partials<2>(wg, acc, {part_rr, part_bb});
 }
 // Factor preconditioner M^-1 = G^T G, G block lower-triangular.  F holds both products'
 // blocks in the matrix's entry order, interleaved: entry (i, j) is G_ij for j <= i and G_ji^T
@@ -319,75 +342,8 @@ __global__ void factor_entries(int V, const int* __restrict__ rowptr, const int*
 #pragma unroll
         for (int k = 0; k < 9; ++k) v[k] = g[k];
 #pragma unroll
-        for (int k = 0; k < 9; ++k) F[il_index(e, k)] = (T)(e <= d ? v[k] : v[3 * (k % 3) + k / 3]);
+        for (int k = 0; k < 9; ++k) F[il_index<T>(e, k)] = (T)(e <= d ? v[k] : v[3 * (k % 3) + k / 3]);
     }
-}
-// row a's part of G r (entries up to the diagonal at d)
-template <typename T, typename X>
-__device__ inline void lower_product(int a, int sub, int e0, int d, const int* __restrict__ col, const T* __restrict__ F,
-                                     const X* __restrict__ x, double y[3]) {
-    y[0] = y[1] = y[2] = 0.0;
-    for (int e = e0 + sub; e <= d; e += kGL) {
-        double w[3];
-        block_mv_il(F, (size_t)e, x + 3 * (size_t)col[e], w);
-        y[0] += w[0]; y[1] += w[1]; y[2] += w[2];
-    }
-    group_reduce3<T>(y);
-}
-// row a's part of G^T t: the diagonal block transposed, the entries above it as stored
-template <typename T, typename X>
-__device__ inline void upper_product(int a, int sub, int d, int e1, const int* __restrict__ col, const T* __restrict__ F,
-                                     const X* __restrict__ x, double y[3]) {
-    y[0] = y[1] = y[2] = 0.0;
-    for (int e = d + sub; e < e1; e += kGL) {
-        const T* b = F + ((size_t)e / kGL) * (9 * kGL) + e % kGL;
-        const X* xe = x + 3 * (size_t)col[e];
-        const int s = e == d ? kGL : 3 * kGL, c = e == d ? 3 * kGL : kGL;   // row and column strides
-        y[0] += (double)b[0] * xe[0] + (double)b[c] * xe[1] + (double)b[2 * c] * xe[2];
-        y[1] += (double)b[s] * xe[0] + (double)b[s + c] * xe[1] + (double)b[s + 2 * c] * xe[2];
-        y[2] += (double)b[2 * s] * xe[0] + (double)b[2 * s + c] * xe[1] + (double)b[2 * s + 2 * c] * xe[2];
-    }
-    group_reduce3<T>(y);
-}
-// t = G r
-template <typename T>
-__global__ __launch_bounds__(kPB) void prec_g1(Layout L, const int* __restrict__ rowptr, const int* __restrict__ dpos,
-                                               const int* __restrict__ col, const T* __restrict__ F, const T* __restrict__ r,
-                                               T* __restrict__ t, const PcgScalars* __restrict__ sc) {
-    int scene, row0, rend;
-    L.block(scene, row0, rend);
-    if (sc && sc[scene].done) return;
-    const int a = row0 + threadIdx.x / kGL, sub = threadIdx.x % kGL;
-    if (a >= rend) return;
-    double y[3];
-    lower_product(a, sub, rowptr[a], dpos[a], col, F, r, y);
-    if (sub == 0)
-        for (int k = 0; k < 3; ++k) t[3 * a + k] = (T)y[k];
-}
-// z = G^T t; partial of r.z; p = z when `init`
-template <typename T>
-__global__ __launch_bounds__(kPB) void prec_g2(Layout L, const int* __restrict__ rowptr, const int* __restrict__ dpos,
-                                               const int* __restrict__ col, const T* __restrict__ F, const T* __restrict__ t,
-                                               const T* __restrict__ r, T* __restrict__ z, T* __restrict__ p, int init,
-                                               const PcgScalars* __restrict__ sc, double* __restrict__ part_rz) {
-    int scene, row0, rend;
-    L.block(scene, row0, rend);
-    if (sc && sc[scene].done) return;
-    const int a = row0 + threadIdx.x / kGL, sub = threadIdx.x % kGL;
-    double acc[1] = {0.0};
-    if (a < rend) {
-        double y[3];
-        upper_product(a, sub, dpos[a], rowptr[a + 1], col, F, t, y);
-        if (sub == 0) {
-            const T zt[3] = {(T)y[0], (T)y[1], (T)y[2]};
-            for (int k = 0; k < 3; ++k) {
-                z[3 * a + k] = zt[k];
-                if (init) p[3 * a + k] = zt[k];
-            }
-            acc[0] = (double)r[3 * a] * zt[0] + (double)r[3 * a + 1] * zt[1] + (double)r[3 * a + 2] * zt[2];
-        }
-    }
-    group_partials<1>(acc, part_rz);
 }
 // Per-scene controls of a batch solve (null for one system): relative tolerance, iteration
 // cap and whether the scene takes part at all.
@@ -404,120 +360,340 @@ __global__ __launch_bounds__(kPB) void pcg_init_scalars(Layout L, const double* 
     const int k = blockIdx.x;
     int lo, n;
     L.parts(k, lo, n);
-    const double rz = sum_partials_fixed(part_rz + lo, n);
-    const double rr = sum_partials_fixed(part_rr + lo, n);
-    const double bb = sum_partials_fixed(part_bb + lo, n);
+    double v[3];
+    sum_partials_fixed<3>({part_rz + lo, part_rr + lo, part_bb + lo}, n, v);
     if (threadIdx.x == 0) {
         const double tol = ctl.rel_tol ? ctl.rel_tol[k] : rel_tol;
         PcgScalars& s = sc[k];
-        s.rz = rz;
-        s.rr = rr;
-        s.bn = sqrt(bb);
-        s.tol = tol * (rel_to_r0 ? sqrt(rr) : sqrt(bb));
-        s.done = !(sqrt(rr) > s.tol) || !(rz > 0.0) || (ctl.active && !ctl.active[k]);
+        s.rz = v[0];
+        s.rr = v[1];
+        s.bn = sqrt(v[2]);
+        s.tol = tol * (rel_to_r0 ? sqrt(v[1]) : sqrt(v[2]));
+        s.done = !(sqrt(v[1]) > s.tol) || !(v[0] > 0.0) || (ctl.active && !ctl.active[k]);
         s.iters = 0;
     }
 }
-// q = A p and partials of p.q
+
+// One iteration is three launches with a factor and two with block-Jacobi, one per true
+// dependency:
+//   pcg_product  beta and the convergence test from the r.z and r.r partials; q = A p
+//   pcg_update   alpha from the p.q partials; x += alpha p, r -= alpha q; t = G r or z = M^-1 r
+//   pcg_factor   z = G^T t
+// What used to be launches of their own is folded into these: the scalars are added up by every
+// work-group from the partials (a scene of more than kOwnSums work-groups, where that read
+// grows past the launch it saves, has pcg_sums do it), and a vector that a product gathers is
+// combined where it is read, p = z + beta p_old and r = r_old - alpha q, so that no launch
+// waits for the update.  Old and new p and r, and the scalars, therefore alternate between two
+// buffers.  A vertex's z and p (and r and q) lie in one 8-component record and t in one of 4:
+// a gather is three 16-byte loads in FP64 and two in FP32 where six 8- or 4-byte ones were,
+// since what bounds these kernels is how many scattered lane loads a CU issues, not bytes.
+// Against one launch per step, replayed as a graph of 16 iterations (us an iteration): four 20^3
+// cubes in contact (37,044 rows) block FSAI 43.5 -> 34.3 FP64, 40 -> 25 FP32, block-Jacobi
+// 28.9 -> 20.8; two 9^3 cubes (2,000 rows) block FSAI 18.5 -> 12.5, block-Jacobi 16.2 -> 8.9.
+// Without the graph's capture a solve also starts sooner: block-Jacobi set-up 0.56 -> 0.12 ms.
+// At 37,044 rows and FP64 the three take 10.8, 10.7 and 7.8 us (about 4 us each when empty):
+// 34.6, 18.5 and 18.5 MB of blocks out of the last-level cache and the gathers' lane loads.
 template <typename T>
-__global__ __launch_bounds__(kPB) void pcg_spmv(Layout L, const int* __restrict__ rowptr, const int* __restrict__ col,
-                                                const T* __restrict__ val, const T* __restrict__ p, T* __restrict__ q,
-                                                const PcgScalars* __restrict__ sc, double* __restrict__ part_pq) {
+struct PcgArgs {
+    Layout L;
+    int S, own_sums;
+    const int *rowptr, *dpos, *col;
+    const T *A, *F, *minv;
+    const double* b;
+    T *x, *zp[2], *rq[2], *t;
+    double *part_pq, *part_rz, *part_rr, *part_bb, *sums;   // sums: 3 per scene, of pcg_sums
+    PcgScalars* sc;                                         // two buffers of S
+    int max_iter;
+    SceneControl ctl;
+    int* active;                                            // scenes not yet done
+    volatile int* host;                                     // pinned: iterations begun, every scene done
+};
+// the two 3-vectors of an 8-component record, the one of a 4-component record
+template <typename T>
+__device__ inline void load_pair(const T* __restrict__ v, T a[3], T b[3]) {
+    using V = typename Wide<T>::type;
+    constexpr int W = 16 / (int)sizeof(T);
+    T f[8];
+#pragma unroll
+    for (int j = 0; j < (W == 2 ? 3 : 2); ++j) {
+        const V t = reinterpret_cast<const V*>(v)[j];
+#pragma unroll
+        for (int i = 0; i < W; ++i) f[j * W + i] = t[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) { a[i] = f[i]; b[i] = f[3 + i]; }
+}
+template <typename T>
+__device__ inline void load_one(const T* __restrict__ v, T a[3]) {
+    using V = typename Wide<T>::type;
+    constexpr int W = 16 / (int)sizeof(T);
+    const V t = *reinterpret_cast<const V*>(v);
+    a[0] = t[0]; a[1] = t[1];
+    if constexpr (W == 2) a[2] = v[2];
+    else a[2] = t[2];
+}
+// Sum over entries e = s, s + kGL, ... < end of B_e v_e.  begin() puts the gathers and blocks of
+// the first STEPS entries in flight (they need no scalar, so a kernel calls it before it adds
+// up the partials), finish() multiplies and goes on, STEPS entries at a time.
+template <typename T, int STEPS, typename Gather, typename Block>
+struct RowProduct {
+    typename Gather::raw v[STEPS];
+    T f[STEPS][9];
+    int s, end;
+    __device__ void load(const Gather& gather, const Block& block) {
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i)
+            if (s + i * kGL < end) {
+                gather.load(s + i * kGL, v[i]);
+                block(s + i * kGL, f[i]);
+            }
+    }
+    __device__ void begin(int first, int last, const Gather& gather, const Block& block) {
+        s = first;
+        end = last;
+        load(gather, block);
+    }
+    __device__ void finish(const Gather& gather, const Block& block, double c, double y[3]) {
+        y[0] = y[1] = y[2] = 0.0;
+        while (s < end) {
+#pragma unroll
+            for (int i = 0; i < STEPS; ++i)
+                if (s + i * kGL < end) {
+                    T w[3];
+                    gather.combine(v[i], c, w);
+#pragma unroll
+                    for (int u = 0; u < 3; ++u)
+                        y[u] += (double)f[i][3 * u] * w[0] + (double)f[i][3 * u + 1] * w[1] + (double)f[i][3 * u + 2] * w[2];
+                }
+            s += STEPS * kGL;
+            load(gather, block);
+        }
+#pragma unroll
+        for (int u = 0; u < 3; ++u) y[u] = row_sum(y[u]);
+    }
+};
+// interleaved blocks; with `transposed` >= 0 that entry's block transposed
+template <typename T>
+struct Blocks {
+    const T* B;
+    int transposed;
+    __device__ void operator()(int e, T f[9]) const {
+        load_block(B + (size_t)(e / kGL) * (9 * kGL), (unsigned)e, f);
+        if (e == transposed) transpose3(f);
+    }
+};
+// first + c second of a record, and the single vector
+template <typename T>
+struct PairGather {
+    struct raw { T a[3], b[3]; };
+    const T* v;
+    const int* col;
+    __device__ void load(int e, raw& r) const { load_pair(v + 8 * (size_t)col[e], r.a, r.b); }
+    __device__ void combine(const raw& r, double c, T w[3]) const {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) w[i] = (T)((double)r.a[i] + c * (double)r.b[i]);
+    }
+};
+template <typename T>
+struct OneGather {
+    struct raw { T a[3]; };
+    const T* v;
+    const int* col;
+    __device__ void load(int e, raw& r) const { load_one(v + 4 * (size_t)col[e], r.a); }
+    __device__ void combine(const raw& r, double, T w[3]) const {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) w[i] = r.a[i];
+    }
+};
+template <typename T>
+__device__ inline T pick3(int sub, const double y[3]) { return (T)(sub == 0 ? y[0] : sub == 1 ? y[1] : y[2]); }
+
+// x = 0, r = b, q = p = 0 (the first direction is z + 0 p); partials of b.b; with block-Jacobi
+// z and the r.z, r.r partials
+template <typename T>
+__global__ __launch_bounds__(kPB) void pcg_start(PcgArgs<T> g) {
+    const int wg = g.L.index();
     int scene, row0, rend;
-    L.block(scene, row0, rend);
-    if (sc[scene].done) return;
+    g.L.block(wg, scene, row0, rend);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *g.active = g.S;
     const int a = row0 + threadIdx.x / kGL, sub = threadIdx.x % kGL;
+    double v[3] = {0, 0, 0};
+    if (a < rend && sub < 3) {
+        const double bv = g.b[3 * (size_t)a + sub];
+        const T r = (T)bv;
+        g.x[3 * (size_t)a + sub] = (T)0;
+        g.rq[0][8 * (size_t)a + sub] = r;
+        g.rq[0][8 * (size_t)a + 3 + sub] = (T)0;
+        g.zp[0][8 * (size_t)a + 3 + sub] = (T)0;
+        v[2] = bv * bv;
+        if (g.minv) {
+            const T* m = g.minv + 9 * (size_t)a + 3 * sub;
+            const double* b = g.b + 3 * (size_t)a;
+            const T z = (T)((double)m[0] * (T)b[0] + (double)m[1] * (T)b[1] + (double)m[2] * (T)b[2]);
+            g.zp[0][8 * (size_t)a + sub] = z;
+            v[0] = (double)r * z;
+            v[1] = (double)r * r;
+        }
+    }
+    group_partials<3>(wg, v, {g.part_rz, g.part_rr, g.part_bb});
+}
+// the scenes' sums of the previous launch's partials (K = 1: p.q; 2: r.z and r.r), one
+// work-group per scene
+template <int K>
+__global__ __launch_bounds__(kPB) void pcg_sums(Layout L, const double* __restrict__ pa, const double* __restrict__ pb, double* __restrict__ sums) {
+    int lo, n;
+    L.parts(blockIdx.x, lo, n);
+    double v[2] = {0, 0};
+    if constexpr (K == 1) {
+        double one[1];
+        sum_partials_fixed<1>({pa + lo}, n, one);
+        v[0] = one[0];
+    } else {
+        sum_partials_fixed<2>({pa + lo, pb + lo}, n, v);
+    }
+    if (threadIdx.x == 0)
+        for (int k = 0; k < K; ++k) sums[3 * blockIdx.x + (K == 1 ? 0 : 1 + k)] = v[k];
+}
+template <typename T>
+__global__ __launch_bounds__(kPB) void pcg_product(PcgArgs<T> g, int it) {
+    const int wg = g.L.index();
+    int scene, row0, rend, lo, n;
+    g.L.block(wg, scene, row0, rend);
+    g.L.parts(scene, lo, n);
+    const int cur = it & 1;
+    PcgScalars s = g.sc[cur * g.S + scene];
+    const int a = row0 + threadIdx.x / kGL, sub = threadIdx.x % kGL;
+    const T* zp = g.zp[cur];
+    const PairGather<T> gather{zp, g.col};
+    const Blocks<T> block{g.A, -1};
+    RowProduct<T, 2, PairGather<T>, Blocks<T>> prod;
+    T z = (T)0, p = (T)0;
+    if (!s.done && a < rend) {
+        prod.begin(g.rowptr[a] + sub, g.rowptr[a + 1], gather, block);
+        if (sub < 3) { z = zp[8 * (size_t)a + sub]; p = zp[8 * (size_t)a + 3 + sub]; }
+    }
+    bool ended = it == 0 && s.done;
+    double beta = 0.0;
+    if (it > 0 && !s.done) {
+        double v[2];
+        if (g.own_sums) sum_partials_fixed<2>({g.part_rz + lo, g.part_rr + lo}, n, v);
+        else { v[0] = g.sums[3 * scene + 1]; v[1] = g.sums[3 * scene + 2]; }
+        beta = v[0] / s.rz;
+        s.rz = v[0];
+        s.rr = v[1];
+        s.iters += 1;
+        const int cap = g.ctl.max_iter ? g.ctl.max_iter[scene] : g.max_iter;
+        s.done = ended = !(sqrt(v[1]) > s.tol) || s.iters >= cap || !(v[0] > 0.0);
+    }
+    if (threadIdx.x == 0) {
+        if (wg == lo) {
+            g.sc[(cur ^ 1) * g.S + scene] = s;
+            if (ended && atomicSub(g.active, 1) == 1) __hip_atomic_store(g.host + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        if (wg == 0) __hip_atomic_store(g.host, it + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (s.done) return;
     double acc[1] = {0.0};
     if (a < rend) {
         double y[3];
-        row_product<T, T>(a, sub, rowptr, col, val, p, y);
-        if (sub == 0) {
-            const T yt[3] = {(T)y[0], (T)y[1], (T)y[2]};
-            for (int k = 0; k < 3; ++k) q[3 * a + k] = yt[k];
-            acc[0] = (double)p[3 * a] * yt[0] + (double)p[3 * a + 1] * yt[1] + (double)p[3 * a + 2] * yt[2];
+        prod.finish(gather, block, beta, y);
+        if (sub < 3) {
+            p = (T)((double)z + beta * (double)p);
+            const T q = pick3<T>(sub, y);
+            g.zp[cur ^ 1][8 * (size_t)a + 3 + sub] = p;
+            g.rq[cur][8 * (size_t)a + 3 + sub] = q;
+            acc[0] = (double)p * (double)q;
         }
     }
-    group_partials<1>(acc, part_pq);
+    group_partials<1>(wg, acc, {g.part_pq});
 }
-// p.q of every scene from the product's partials, once (one work-group per scene)
-__global__ __launch_bounds__(kPB) void pcg_reduce_pq(Layout L, const double* __restrict__ part_pq, PcgScalars* __restrict__ sc) {
-    const int k = blockIdx.x;
-    if (sc[k].done) return;
-    int lo, n;
-    L.parts(k, lo, n);
-    const double pq = sum_partials_fixed(part_pq + lo, n);
-    if (threadIdx.x == 0) sc[k].pq = pq;
+// it < 0: the start's t = G r
+template <typename T, bool FACTOR>
+__global__ __launch_bounds__(kPB) void pcg_update(PcgArgs<T> g, int it) {
+    const int wg = g.L.index();
+    int scene, row0, rend, lo, n;
+    g.L.block(wg, scene, row0, rend);
+    g.L.parts(scene, lo, n);
+    const int cur = it < 0 ? 0 : it & 1;
+    PcgScalars s;
+    if (it >= 0) {
+        s = g.sc[(cur ^ 1) * g.S + scene];
+        if (s.done) return;
+    }
+    const int a = row0 + threadIdx.x / kGL, sub = threadIdx.x % kGL;
+    const PairGather<T> gather{g.rq[cur], g.col};
+    const Blocks<T> block{g.F, -1};
+    RowProduct<T, 2, PairGather<T>, Blocks<T>> prod;
+    T x = (T)0, p = (T)0, r = (T)0, q = (T)0, m[3] = {(T)0, (T)0, (T)0};
+    if (a < rend) {
+        if (FACTOR) prod.begin(g.rowptr[a] + sub, g.dpos[a] + 1, gather, block);
+        if (it >= 0 && sub < 3) {
+            const T* rq = g.rq[cur] + 8 * (size_t)a + sub;
+            x = g.x[3 * (size_t)a + sub];
+            p = g.zp[cur ^ 1][8 * (size_t)a + 3 + sub];
+            r = rq[0];
+            q = rq[3];
+            if (!FACTOR)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) m[i] = g.minv[9 * (size_t)a + 3 * sub + i];
+        }
+    }
+    double alpha = 0.0;
+    if (it >= 0) {
+        double v[1];
+        if (g.own_sums) sum_partials_fixed<1>({g.part_pq + lo}, n, v);
+        else v[0] = g.sums[3 * scene];
+        alpha = s.rz / v[0];
+    }
+    double acc[2] = {0.0, 0.0};
+    if (a < rend) {
+        if (it >= 0 && sub < 3) {
+            g.x[3 * (size_t)a + sub] = (T)((double)x + alpha * (double)p);
+            r = (T)((double)r - alpha * (double)q);
+            g.rq[cur ^ 1][8 * (size_t)a + sub] = r;
+        }
+        if (FACTOR) {
+            double y[3];
+            prod.finish(gather, block, -alpha, y);
+            if (sub < 3) g.t[4 * (size_t)a + sub] = pick3<T>(sub, y);
+        } else {
+            const T r0 = __shfl(r, 0, kGL), r1 = __shfl(r, 1, kGL), r2 = __shfl(r, 2, kGL);
+            if (sub < 3) {
+                const T z = (T)((double)m[0] * r0 + (double)m[1] * r1 + (double)m[2] * r2);
+                g.zp[cur ^ 1][8 * (size_t)a + sub] = z;
+                acc[0] = (double)r * (double)z;
+                acc[1] = (double)r * (double)r;
+            }
+        }
+    }
+    if (!FACTOR) group_partials<2>(wg, acc, {g.part_rz, g.part_rr});
 }
-// alpha = rz / p.q; x += alpha p; r -= alpha q; partial of r.r; with block-Jacobi (minv set)
-// also z = M^-1 r and its r.z partial
 template <typename T>
-__global__ __launch_bounds__(kPB) void pcg_update(Layout L, const T* __restrict__ minv,
-                                                  const T* __restrict__ p, const T* __restrict__ q, T* __restrict__ x, T* __restrict__ r,
-                                                  T* __restrict__ z, const PcgScalars* __restrict__ sc, double* __restrict__ part_rz,
-                                                  double* __restrict__ part_rr) {
+__global__ __launch_bounds__(kPB) void pcg_factor(PcgArgs<T> g, int it) {
+    const int wg = g.L.index();
     int scene, row0, rend;
-    L.block(scene, row0, rend);
-    if (sc[scene].done) return;
-    const double alpha = sc[scene].rz / sc[scene].pq;
+    g.L.block(wg, scene, row0, rend);
+    const int to = it < 0 ? 0 : (it & 1) ^ 1;
+    if (it >= 0 && g.sc[to * g.S + scene].done) return;
     const int a = row0 + threadIdx.x / kGL, sub = threadIdx.x % kGL;
     double acc[2] = {0.0, 0.0};
-    if (a < rend && sub == 0) {
-        T rt[3];
-        for (int k = 0; k < 3; ++k) {
-            x[3 * a + k] = (T)((double)x[3 * a + k] + alpha * (double)p[3 * a + k]);
-            rt[k] = (T)((double)r[3 * a + k] - alpha * (double)q[3 * a + k]);
-            r[3 * a + k] = rt[k];
+    if (a < rend) {
+        const int d = g.dpos[a];
+        const OneGather<T> gather{g.t, g.col};
+        const Blocks<T> block{g.F, d};   // the diagonal block is stored as G_aa
+        RowProduct<T, 2, OneGather<T>, Blocks<T>> prod;
+        prod.begin(d + sub, g.rowptr[a + 1], gather, block);
+        const T r = sub < 3 ? g.rq[to][8 * (size_t)a + sub] : (T)0;
+        double y[3];
+        prod.finish(gather, block, 0.0, y);
+        if (sub < 3) {
+            const T z = pick3<T>(sub, y);
+            g.zp[to][8 * (size_t)a + sub] = z;
+            acc[0] = (double)r * (double)z;
+            acc[1] = (double)r * (double)r;
         }
-        if (minv) {
-            double zv[3];
-            block_mv(minv + (size_t)9 * a, rt, zv);
-            for (int k = 0; k < 3; ++k) z[3 * a + k] = (T)zv[k];
-            acc[0] = (double)rt[0] * (T)zv[0] + (double)rt[1] * (T)zv[1] + (double)rt[2] * (T)zv[2];
-        }
-        acc[1] = (double)rt[0] * rt[0] + (double)rt[1] * rt[1] + (double)rt[2] * rt[2];
     }
-    if (minv) group_partials2(acc, part_rz, part_rr);
-    else { double a1[1] = {acc[1]}; group_partials<1>(a1, part_rr); }
-}
-// p = z + beta p with the beta of pcg_scalars (one DOF per thread); skipped by a scene that
-// has just converged, whose direction is no longer used
-template <typename T>
-__global__ __launch_bounds__(kPB) void pcg_direction(int V, const T* __restrict__ z, T* __restrict__ p, const PcgScalars* __restrict__ sc) {
-    if (sc->done) return;
-    const double beta = sc->beta;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;       // one DOF per thread
-    if (t < 3 * V) p[t] = (T)((double)z[t] + beta * (double)p[t]);
-}
-// the same on the row layout of a batch: the 3 kRows DOFs of the work-group's rows
-template <typename T>
-__global__ __launch_bounds__(kPB) void pcg_direction_rows(Layout L, const T* __restrict__ z, T* __restrict__ p,
-                                                          const PcgScalars* __restrict__ sc) {
-    int scene, row0, rend;
-    L.block(scene, row0, rend);
-    if (sc[scene].done) return;
-    const double beta = sc[scene].beta;
-    const int t = 3 * row0 + threadIdx.x;
-    if ((int)threadIdx.x < 3 * kRows && t < 3 * rend) p[t] = (T)((double)z[t] + beta * (double)p[t]);
-}
-// r.z', r.r and beta = r.z' / r.z from the partials, once per iteration (one work-group per
-// scene); the convergence test
-__global__ void pcg_scalars(Layout L, const double* __restrict__ part_rz, const double* __restrict__ part_rr,
-                            PcgScalars* __restrict__ sc, int max_iter, SceneControl ctl) {
-    const int k = blockIdx.x;
-    if (sc[k].done) return;
-    int lo, n;
-    L.parts(k, lo, n);
-    const double rz1 = sum_partials_fixed(part_rz + lo, n);
-    const double rr = sum_partials_fixed(part_rr + lo, n);
-    if (threadIdx.x == 0) {
-        PcgScalars& s = sc[k];
-        const int cap = ctl.max_iter ? ctl.max_iter[k] : max_iter;
-        s.beta = rz1 / s.rz;
-        s.rz = rz1;
-        s.rr = rr;
-        s.iters += 1;
-        if (!(sqrt(rr) > s.tol) || s.iters >= cap || !(rz1 > 0.0)) s.done = 1;
-    }
+    group_partials<2>(wg, acc, {g.part_rz, g.part_rr});
 }
 // x (FP64) += d (FP32), for the refinement (scenes with add[scene] != 0 when add is set)
 __global__ void add_correction(int n, const float* __restrict__ d, double* __restrict__ x, const int* __restrict__ vs,
@@ -525,13 +701,10 @@ __global__ void add_correction(int n, const float* __restrict__ d, double* __res
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n && (!add || add[vs[i / 3]])) x[i] += (double)d[i];
 }
-__global__ void zero_d(int n, double* __restrict__ x) {
+template <typename T>
+__global__ void zero_v(int n, T* __restrict__ x) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[i] = 0.0;
-}
-__global__ void zero_f(int n, float* __restrict__ x) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[i] = 0.0f;
+    if (i < n) x[i] = (T)0;
 }
 
 // ---- block FSAI factor ----------------------------------------------------------------
@@ -719,12 +892,6 @@ void read_scalars(Context& c, const PcgScalars* d, int S, std::vector<PcgScalars
     h.resize(S);
     read_back(c, h.data(), d, (size_t)S);
 }
-bool all_done(const std::vector<PcgScalars>& h) {
-    for (const PcgScalars& s : h)
-        if (!s.done) return false;
-    return true;
-}
-
 // The preconditioner of one solve: block-Jacobi (minv) or a factor (F, factor_entries).
 template <typename T>
 struct Prec {
@@ -765,72 +932,73 @@ Layout make_layout(Context& c) {
     return L;
 }
 
+// PCG solves of A x = b from x = 0 (b FP64; A, x and the work vectors in T), one per scene in
+// lock step.  The host keeps at most kAhead iterations enqueued beyond the one that the device
+// last began, so that few launches follow the last scene's convergence.  Returns the scenes'
+// final scalars.
 template <typename T>
-void apply_prec(Context& c, const Layout& L, const Prec<T>& M, const T* r, T* z, T* p, int init, const PcgScalars* sc, double* part_rz) {
+void pcg_run(Context& c, const Layout& L, int S, const T* val, const Prec<T>& M, const double* b, T* x, double rel_tol, int rel_to_r0,
+             int max_iter, SceneControl ctl, std::vector<PcgScalars>& h) {
+    const size_t V = (size_t)c.sc.V;
     SolveBuffers& w = c.solve;
-    if (M.F) {
-        T* t = reinterpret_cast<T*>(w.t.p);
-        hipLaunchKernelGGL(prec_g1<T>, dim3(L.ng), dim3(kPB), 0, c.stream, L, w.rowptr.p, w.dpos.p, w.col.p, M.F, r, t, sc);
-        hipLaunchKernelGGL(prec_g2<T>, dim3(L.ng), dim3(kPB), 0, c.stream, L, w.rowptr.p, w.dpos.p, w.col.p, M.F, t, r, z, p, init, sc,
-                           part_rz);
-    } else {
-        hipLaunchKernelGGL(prec_jacobi<T>, dim3(L.ng), dim3(kPB), 0, c.stream, L, M.minv, r, z, p, init, sc, part_rz);
+    w.zp.resize(16 * V); w.rq.resize(16 * V); w.t.resize(4 * V);
+    w.sums.resize(3 * (size_t)S);
+    w.active.resize(1);
+    c.pin_pcg.reserve(2);
+    PcgArgs<T> g;
+    g.L = L; g.S = S;
+    int most = L.ng;
+    if (S > 1) {
+        most = 0;
+        for (int k = 0; k < S; ++k) most = std::max(most, (int)blocks_for((size_t)(c.sc.h_voff[k + 1] - c.sc.h_voff[k]), kRows));
     }
-}
-
-// PCG solves of A x = b (b FP64; A, x and the work vectors in T), one per scene in lock step.
-// kCheck iterations are captured once into a HIP graph and replayed until the device flags
-// say that every scene has converged.  Returns the scenes' final scalars.
-template <typename T>
-void pcg_run(Context& c, const Layout& L, int S, const T* val, const Prec<T>& M, const double* b, T* x, int x_zero, double rel_tol,
-             int rel_to_r0, int max_iter, SceneControl ctl, std::vector<PcgScalars>& h) {
-    const int V = c.sc.V;
-    const int ng = L.ng;
-    const int ngd = (int)blocks_for(3 * V, kPB);
-    SolveBuffers& w = c.solve;
-    T* r = reinterpret_cast<T*>(w.r.p);
-    T* z = reinterpret_cast<T*>(w.z.p);
-    T* p = reinterpret_cast<T*>(w.p.p);
-    T* q = reinterpret_cast<T*>(w.q.p);
-    double* part_pq = w.part.p;
-    double* part_rz = w.part.p + ng;
-    double* part_rr = w.part.p + 2 * ng;
-    double* part_bb = w.part.p + 3 * ng;
-    PcgScalars* sc = reinterpret_cast<PcgScalars*>(w.scal.p);
-    hipLaunchKernelGGL(pcg_residual<T>, dim3(ng), dim3(kPB), 0, c.stream, L, w.rowptr.p, w.col.p, val, b, x, x_zero, r, part_rr, part_bb);
-    apply_prec<T>(c, L, M, r, z, p, 1, nullptr, part_rz);
-    hipLaunchKernelGGL(pcg_init_scalars, dim3(S), dim3(kPB), 0, c.stream, L, part_rz, part_rr, part_bb, rel_tol, rel_to_r0, ctl, sc);
+    g.own_sums = most <= kOwnSums;
+    g.rowptr = w.rowptr.p; g.dpos = w.dpos.p; g.col = w.col.p;
+    g.A = val; g.F = M.F; g.minv = M.minv; g.b = b; g.x = x;
+    for (int i = 0; i < 2; ++i) {
+        g.zp[i] = reinterpret_cast<T*>(w.zp.p) + 8 * V * i;
+        g.rq[i] = reinterpret_cast<T*>(w.rq.p) + 8 * V * i;
+    }
+    g.t = reinterpret_cast<T*>(w.t.p);
+    g.part_pq = w.part.p; g.part_rz = w.part.p + L.ng; g.part_rr = w.part.p + 2 * (size_t)L.ng; g.part_bb = w.part.p + 3 * (size_t)L.ng;
+    g.sums = w.sums.p;
+    g.sc = reinterpret_cast<PcgScalars*>(w.scal.p);
+    g.max_iter = max_iter; g.ctl = ctl;
+    g.active = w.active.p;
+    g.host = c.pin_pcg.p;
+    volatile int* host = c.pin_pcg.p;
+    host[0] = host[1] = 0;
+    const dim3 rows(L.ng), threads(kPB);
+    hipLaunchKernelGGL(pcg_start<T>, rows, threads, 0, c.stream, g);
+    if (g.F) {
+        hipLaunchKernelGGL((pcg_update<T, true>), rows, threads, 0, c.stream, g, -1);
+        hipLaunchKernelGGL(pcg_factor<T>, rows, threads, 0, c.stream, g, -1);
+    }
+    hipLaunchKernelGGL(pcg_init_scalars, dim3(S), threads, 0, c.stream, L, g.part_rz, g.part_rr, g.part_bb, rel_tol, rel_to_r0, ctl, g.sc);
     CIPC_CHECK_LAUNCH();
-    read_scalars(c, sc, S, h);
-    if (all_done(h)) return;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    CIPC_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < kCheck; ++k) {
-        hipLaunchKernelGGL(pcg_spmv<T>, dim3(ng), dim3(kPB), 0, c.stream, L, w.rowptr.p, w.col.p, val, p, q, sc, part_pq);
-        hipLaunchKernelGGL(pcg_reduce_pq, dim3(S), dim3(kPB), 0, c.stream, L, part_pq, sc);
-        hipLaunchKernelGGL(pcg_update<T>, dim3(ng), dim3(kPB), 0, c.stream, L, M.F ? nullptr : M.minv, p, q, x, r, z, sc,
-                           part_rz, part_rr);
-        if (M.F) apply_prec<T>(c, L, M, r, z, p, 0, sc, part_rz);
-        hipLaunchKernelGGL(pcg_scalars, dim3(S), dim3(kPB), 0, c.stream, L, part_rz, part_rr, sc, max_iter, ctl);
-        if (L.bl) hipLaunchKernelGGL(pcg_direction_rows<T>, dim3(ng), dim3(kPB), 0, c.stream, L, z, p, sc);
-        else hipLaunchKernelGGL(pcg_direction<T>, dim3(ngd), dim3(kPB), 0, c.stream, V, z, p, sc);
-    }
-    const hipError_t ce = hipStreamEndCapture(c.stream, &graph);
-    CIPC_HIP(ce);
-    CIPC_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-    try {
-        while (!all_done(h)) {
-            CIPC_HIP(hipGraphLaunch(exec, c.stream));
-            read_scalars(c, sc, S, h);
+    int it = 0;
+    for (unsigned spins = 0; !host[1];) {
+        if (it - host[0] >= kAhead) {
+            // a failed launch or a lost device never reports: asked now and then
+            if ((++spins & 0xfffff) == 0 && hipStreamQuery(c.stream) != hipErrorNotReady && it - host[0] >= kAhead && !host[1]) {
+                CIPC_HIP(hipStreamSynchronize(c.stream));
+                throw Error(CIPC_ERR_HIP, "the conjugate-gradient iteration stopped reporting");
+            }
+            continue;
         }
-    } catch (...) {
-        (void)hipGraphExecDestroy(exec);
-        (void)hipGraphDestroy(graph);
-        throw;
+        hipLaunchKernelGGL(pcg_product<T>, rows, threads, 0, c.stream, g, it);
+        if (!g.own_sums) hipLaunchKernelGGL(pcg_sums<1>, dim3(S), threads, 0, c.stream, L, g.part_pq, (const double*)nullptr, g.sums);
+        if (g.F) {
+            hipLaunchKernelGGL((pcg_update<T, true>), rows, threads, 0, c.stream, g, it);
+            hipLaunchKernelGGL(pcg_factor<T>, rows, threads, 0, c.stream, g, it);
+        } else {
+            hipLaunchKernelGGL((pcg_update<T, false>), rows, threads, 0, c.stream, g, it);
+        }
+        if (!g.own_sums) hipLaunchKernelGGL(pcg_sums<2>, dim3(S), threads, 0, c.stream, L, g.part_rz, g.part_rr, g.sums);
+        CIPC_CHECK_LAUNCH();
+        ++it;
     }
-    (void)hipGraphExecDestroy(exec);
-    (void)hipGraphDestroy(graph);
+    read_scalars(c, g.sc + (size_t)(it & 1) * S, S, h);
 }
 
 // Per-scene state of the FP64 refinement.
@@ -893,9 +1061,8 @@ void linear_solve_scenes(Context& c, int precision, int preconditioner, double r
     SolveBuffers& w = c.solve;
     const Layout L = make_layout(c);
     const int ng = L.ng;
-    w.r.resize((size_t)n); w.z.resize((size_t)n); w.p.resize((size_t)n); w.q.resize((size_t)n); w.t.resize((size_t)n);
     w.part.resize((size_t)4 * ng);
-    w.scal.resize((size_t)S * ((sizeof(PcgScalars) + 7) / 8));
+    w.scal.resize(2 * (size_t)S * ((sizeof(PcgScalars) + 7) / 8));
     w.x.resize((size_t)n);
     const bool fp32 = precision == 1;
     build_solve_matrix(c, fp32, preconditioner == 2);
@@ -947,9 +1114,8 @@ void linear_solve_scenes(Context& c, int precision, int preconditioner, double r
     }
     for (int k = 0; k < S; ++k) res[k] = SolveResult{};
     std::vector<PcgScalars> h;
-    hipLaunchKernelGGL(zero_d, dim3(blocks_for(n, 256)), dim3(256), 0, c.stream, n, w.x.p);
     if (precision == 0) {
-        pcg_run<double>(c, L, S, w.vil.p, Md, c.rhs.p, w.x.p, 1, rel_tol, 0, max_iter, ctl, h);
+        pcg_run<double>(c, L, S, w.vil.p, Md, c.rhs.p, w.x.p, rel_tol, 0, max_iter, ctl, h);
         for (int k = 0; k < S; ++k) {
             res[k].iterations = h[k].iters;
             res[k].rel_residual = h[k].bn > 0 ? std::sqrt(h[k].rr) / h[k].bn : 0.0;
@@ -958,6 +1124,7 @@ void linear_solve_scenes(Context& c, int precision, int preconditioner, double r
         // FP64 refinement around FP32 PCG; each inner solve aims just past the remaining
         // reduction (floored at the FP32 reach), so one or two refinements usually suffice
         w.xf.resize((size_t)n); w.res.resize((size_t)n);
+        hipLaunchKernelGGL(zero_v<double>, dim3(blocks_for(n, 256)), dim3(256), 0, c.stream, n, w.x.p);
         double* part_rr = w.part.p + 2 * ng;
         double* part_bb = w.part.p + 3 * ng;
         PcgScalars* sc = reinterpret_cast<PcgScalars*>(w.scal.p);
@@ -995,9 +1162,8 @@ void linear_solve_scenes(Context& c, int precision, int preconditioner, double r
                 ictl.max_iter = w.ctl_i.p + S;
                 ictl.active = w.ctl_i.p;
             }
-            hipLaunchKernelGGL(zero_f, dim3(blocks_for(n, 256)), dim3(256), 0, c.stream, n, w.xf.p);
             std::vector<PcgScalars> hi;
-            pcg_run<float>(c, L, S, w.vilf.p, Mf, rd, w.xf.p, 1, itol[0], 1, icap[0], ictl, hi);
+            pcg_run<float>(c, L, S, w.vilf.p, Mf, rd, w.xf.p, itol[0], 1, icap[0], ictl, hi);
             // scenes that made no progress (breakdown) or hit the refinement cap stop here,
             // without their correction
             std::fill(add.begin(), add.end(), 0);
