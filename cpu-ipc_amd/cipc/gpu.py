@@ -471,7 +471,7 @@ class GpuContext:
         return {names[e[k].kernel]: (e[k].chosen, list(e[k].ms[:e[k].n_candidates])) for k in range(n.value)}
 
     def set_tune(self, kernel, choice):
-        """kernel 0 / 1: full-CCD walk splits, 3 / 4: the active set's walk splits (2^choice
+        """kernel 0 / 1: full-CCD walk splits, 3 / 4: the active set's walk splits (4 * 2^choice
         lanes per query); kernel 2: the iteration graph off (0) or on (1)."""
         _check(load().cipc_gpu_set_tune(self.h, kernel, choice))
 

@@ -133,86 +133,108 @@ __global__ void partial_ccd_kernel(const int* __restrict__ n_dev, const int2* __
     scene_atomic<false>(sl, scene, 2, a);
 }
 
-// Full CCD, point-triangle phase (ContactMechanics.cpp:3764-3816): each surface vertex is
-// split over 2^pb lanes, one subtree of the swept face tree each; the step is the min
-// over every lane, reduced across the wavefront before one atomic.  The minimum does not
-// depend on the split, which the autotuner picks per context.
+// Full CCD, point-triangle phase (ContactMechanics.cpp:3764-3816): each surface vertex walks the
+// swept face tree with 4 << bits lanes; the pairs it meets are filtered and the rest advanced 64
+// at a time (pair_walk), capped at the step found so far (the cap only ends an advance that
+// cannot lower the minimum).  The minimum does not depend on the order or the lanes per query,
+// which the autotuner picks per context.  An advance takes hundreds of times a record's test and
+// few of the pairs met need one: a lane that advanced its own pairs while it walked held up the
+// other 63.  Alone, on four 20^3 cubes 65 -> 21 us (edges 133 -> 29), four 32^3 256 -> 37
+// (168 -> 52), folded 128^2 cloth 228 -> 34 (505 -> 78), a batch of 40 scenes 147 -> 47 (344 -> 105).
+// The step found so far is read from the slots; an older, larger value is as valid a cap.
+__device__ inline double ccd_cap(const unsigned long long* sl, int scene) {
+    return bits_to_double(__hip_atomic_load(sl + kSlots * scene + 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
 __global__ __launch_bounds__(64) void full_ccd_pt_kernel(int Vs, const int* __restrict__ perm, const int* __restrict__ sv,
                                                           const int4* __restrict__ faces, const int* __restrict__ bt,
                                                           const double* __restrict__ x, const double* __restrict__ p,
-                                                          TreeView tv, unsigned long long* __restrict__ sl, double eta,
-                                                          const int* __restrict__ vs, int pb) {
-    __shared__ int stk[kStack * 64];
-    const int t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    double best = 1.0;
-    int scene = kNoScene;
-    if (t < (Vs << pb)) {
-        const int s = perm[t >> pb], part = t & ((1 << pb) - 1);
-        const int vI = sv[s];
-        scene = scene_of(vs, vI);
-        const double a = bits_to_double(sl[kSlots * scene + 5]);
-        const d3 X = ld3(x, vI), P = ld3(p, vI);
-        const Box vb = swept_pt(X, P, a);   // the query box: the point swept with the trees' step
-        part_walk(tv, part, vb, 0.0, stk + threadIdx.x, [&](int f) {
-            const int4 fv = faces[f];
-            if (is_collider(bt[vI]) && is_collider(bt[fv.x]) && is_collider(bt[fv.y]) && is_collider(bt[fv.z])) return;
-            if (vI == fv.x || vI == fv.y || vI == fv.z) return;
-            if (vs && vs[fv.x] != scene) return;          // scenes of a batch never touch
-            const d3 x0 = ld3(x, fv.x), x1 = ld3(x, fv.y), x2 = ld3(x, fv.z);
-            const d3 p0 = ld3(p, fv.x), p1 = ld3(p, fv.y), p2 = ld3(p, fv.z);
-            const Box fb = box_union(box_union(swept_pt(x0, p0, a), swept_pt(x1, p1, a)), swept_pt(x2, p2, a));
-            if (!overlaps(vb, fb, 0.0)) return;
-            // capped at the lane's best so far, itself at most the seeded step a: the
-            // minimum over all pairs is unchanged
-            const double la = accd_pt(X, x0, x1, x2, -P, -p0, -p1, -p2, eta, 0.0, fmin(best, a));
-            best = fmin(la, best);
-        }, [] {}, pb);
+                                                          TreeView tv, unsigned long long* sl, double eta,
+                                                          const int* __restrict__ vs, int bits) {
+    __shared__ int lds[kWalkInts];
+    __shared__ int2 met[kPairQueue], kept[kPairQueue];
+    const WalkGroup G(bits);
+    const int s = walk_query(G, xcd_block(blockIdx.x, gridDim.x), Vs, perm);
+    int v = -1;
+    Box q{};
+    if (s >= 0) {
+        v = sv[s];
+        q = swept_pt(ld3(x, v), ld3(p, v), bits_to_double(sl[kSlots * scene_of(vs, v) + 5]));   // swept with the trees' step
     }
-    scene_atomic<false>(sl, scene, 3, best);
+    pair_walk<false>(tv, G, v, q, 0, lds, met, kept, [&](int2 pr) {
+        const int vI = pr.x;
+        const int4 fv = faces[pr.y];
+        if (is_collider(bt[vI]) && is_collider(bt[fv.x]) && is_collider(bt[fv.y]) && is_collider(bt[fv.z])) return false;
+        if (vI == fv.x || vI == fv.y || vI == fv.z) return false;
+        const int scene = scene_of(vs, vI);
+        if (vs && vs[fv.x] != scene) return false;          // scenes of a batch never touch
+        const double a = bits_to_double(sl[kSlots * scene + 5]);
+        const Box vb = swept_pt(ld3(x, vI), ld3(p, vI), a);
+        const Box fb = box_union(box_union(swept_pt(ld3(x, fv.x), ld3(p, fv.x), a), swept_pt(ld3(x, fv.y), ld3(p, fv.y), a)),
+                                 swept_pt(ld3(x, fv.z), ld3(p, fv.z), a));
+        return overlaps(vb, fb, 0.0);
+    }, [&](bool on, int2 pr) {
+        double la = 1.0;
+        int scene = kNoScene;
+        if (on) {
+            const int vI = pr.x;
+            const int4 fv = faces[pr.y];
+            const int sc = scene_of(vs, vI);
+            const double cap = fmin(bits_to_double(sl[kSlots * sc + 5]), ccd_cap(sl, sc));
+            la = accd_pt(ld3(x, vI), ld3(x, fv.x), ld3(x, fv.y), ld3(x, fv.z), -ld3(p, vI), -ld3(p, fv.x), -ld3(p, fv.y), -ld3(p, fv.z),
+                         eta, 0.0, cap);
+            if (la < cap) scene = sc;
+        }
+        scene_atomic<false>(sl, scene, 3, la);
+    });
 }
 
 // Full CCD, edge-edge phase (ContactMechanics.cpp:3818-3866): every unordered pair of
 // surface edges whose swept boxes (built with the incoming step) overlap, the pair ordered as
 // the reference orders it (I the larger edge id, J the smaller) and filtered with the exact
-// swept boxes of the point-triangle-reduced step read from the slots.  Each edge (split over
-// 2^pb lanes) walks only the leaves after its own leaf, so each pair is met once.
+// swept boxes of the point-triangle-reduced step read from the slots.  Each edge (4 << bits
+// lanes) walks only the leaves after its own leaf, so each pair is met once.
 __global__ __launch_bounds__(64) void full_ccd_ee_kernel(int Es, const int* __restrict__ perm, const int2* __restrict__ se,
                                                           const int* __restrict__ bt, const double* __restrict__ x,
-                                                          const double* __restrict__ p, TreeView tv, const Box* __restrict__ ebox,
-                                                          unsigned long long* __restrict__ sl, double eta, const int* __restrict__ vs,
-                                                          int pb) {
-    __shared__ int stk[kStack * 64];
-    const int t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    double best = 1.0;
-    int scene = kNoScene;
-    if (t < (Es << pb)) {
-        const int eQ = perm[t >> pb], part = t & ((1 << pb) - 1);
-        const int2 Q = se[eQ];
-        scene = scene_of(vs, Q.x);
-        const double a = bits_to_double(sl[kSlots * scene + 4]);
-        const Box bq = box_union(swept_pt(ld3(x, Q.x), ld3(p, Q.x), a), swept_pt(ld3(x, Q.y), ld3(p, Q.y), a));
-        // Query box: bq, swept with the point-triangle-reduced step, which is at most the
-        // tree's step.  The swept box of a smaller step lies inside that of a larger one (the
-        // rounded end point x - a p moves monotonically with a), so bq lies inside the edge's
-        // leaf box and every H's filter box bh inside its leaf box: a pair that passes the
-        // final bq/bh test passes the leaf-box test too, and walking with bq finds it.
-        part_walk_after(tv, part, bq, 0.0, tv.leafpos[eQ], stk + threadIdx.x, [&](int eH) {
-            if (!overlaps(bq, ebox[eH], 0.0)) return;  // exact leaf test (the walk's boxes are float)
-            const int eI = eH > eQ ? eH : eQ, eJ = eH > eQ ? eQ : eH;
-            const int2 I = se[eI], J = se[eJ];
-            if (is_collider(bt[I.x]) && is_collider(bt[I.y]) && is_collider(bt[J.x]) && is_collider(bt[J.y])) return;
-            if (I.x == J.x || I.x == J.y || I.y == J.x || I.y == J.y) return;
-            const int2 H = se[eH];
-            if (vs && vs[H.x] != scene) return;            // scenes of a batch never touch
-            const Box bh = box_union(swept_pt(ld3(x, H.x), ld3(p, H.x), a), swept_pt(ld3(x, H.y), ld3(p, H.y), a));
-            if (!overlaps(bq, bh, 0.0)) return;
-            const d3 i0 = ld3(x, I.x), i1 = ld3(x, I.y), pi0 = ld3(p, I.x), pi1 = ld3(p, I.y);
-            const d3 j0 = ld3(x, J.x), j1 = ld3(x, J.y), pj0 = ld3(p, J.x), pj1 = ld3(p, J.y);
-            const double la = accd_ee(i0, i1, j0, j1, -pi0, -pi1, -pj0, -pj1, eta, 0.0, fmin(best, a));
-            best = fmin(la, best);
-        }, [] {}, pb);
+                                                          const double* __restrict__ p, TreeView tv, unsigned long long* sl,
+                                                          double eta, const int* __restrict__ vs, int bits) {
+    __shared__ int lds[kWalkInts];
+    __shared__ int2 met[kPairQueue], kept[kPairQueue];
+    const WalkGroup G(bits);
+    const int e = walk_query(G, xcd_block(blockIdx.x, gridDim.x), Es, perm);
+    // Query box: swept with the point-triangle-reduced step, which is at most the
+    // tree's step.  The swept box of a smaller step lies inside that of a larger one (the
+    // rounded end point x - a p moves monotonically with a), so it lies inside the edge's
+    // leaf box and every other edge's filter box inside that one's leaf box: a pair that passes
+    // the filter's box test passes the leaf-box test too, and the walk finds it.
+    auto swept = [&](int2 E, double a) { return box_union(swept_pt(ld3(x, E.x), ld3(p, E.x), a), swept_pt(ld3(x, E.y), ld3(p, E.y), a)); };
+    Box q{};
+    int after = 0;
+    if (e >= 0) {
+        const int2 Q = se[e];
+        q = swept(Q, bits_to_double(sl[kSlots * scene_of(vs, Q.x) + 4]));
+        after = tv.leafpos[e];
     }
-    scene_atomic<false>(sl, scene, 3, best);
+    pair_walk<true>(tv, G, e, q, after, lds, met, kept, [&](int2 pr) {
+        const int2 Q = se[pr.x], H = se[pr.y];
+        if (is_collider(bt[Q.x]) && is_collider(bt[Q.y]) && is_collider(bt[H.x]) && is_collider(bt[H.y])) return false;
+        if (Q.x == H.x || Q.x == H.y || Q.y == H.x || Q.y == H.y) return false;
+        const int scene = scene_of(vs, Q.x);
+        if (vs && vs[H.x] != scene) return false;            // scenes of a batch never touch
+        const double a = bits_to_double(sl[kSlots * scene + 4]);
+        return overlaps(swept(Q, a), swept(H, a), 0.0);
+    }, [&](bool on, int2 pr) {
+        double la = 1.0;
+        int scene = kNoScene;
+        if (on) {
+            const int2 I = se[max(pr.x, pr.y)], J = se[min(pr.x, pr.y)];
+            const int sc = scene_of(vs, I.x);
+            const double cap = fmin(bits_to_double(sl[kSlots * sc + 4]), ccd_cap(sl, sc));
+            la = accd_ee(ld3(x, I.x), ld3(x, I.y), ld3(x, J.x), ld3(x, J.y), -ld3(p, I.x), -ld3(p, I.y), -ld3(p, J.x), -ld3(p, J.y), eta,
+                         0.0, cap);
+            if (la < cap) scene = sc;
+        }
+        scene_atomic<false>(sl, scene, 3, la);
+    });
 }
 // slot 4 = slot 3 of every scene: the point-triangle result that the edge-edge phase filters with
 __global__ void copy_pt_result(int S, unsigned long long* sl) {
@@ -270,7 +292,6 @@ void step_bound_early(Context& c, hipStream_t st, bool ground) {
     build_swept_trees(c, sl.p + 5, st);
     LBVH& ft = c.sface_tree;
     LBVH& et = c.sedge_tree;
-    const TreeView ftv{ft.n, ft.nodes.p, ft.wide.p}, etv{et.n, et.nodes.p, et.wide.p, et.leafpos.p};
     if (s.Vs > 0 && ft.n > 0) launch_full_ccd_pt(c, st, c.tune.ccd_pt_bits);
     if (s.Es > 0 && et.n > 0) {
         hipLaunchKernelGGL(copy_pt_result, dim3(blocks_for(S, 64)), dim3(64), 0, st, S, sl.p);
@@ -279,20 +300,20 @@ void step_bound_early(Context& c, hipStream_t st, bool ground) {
     CIPC_CHECK_LAUNCH();
 }
 
-// The two full-CCD walks with each surface vertex / edge split over 2^pb lanes.
+// The two full-CCD walks with 4 << pb lanes per surface vertex / edge.
 void launch_full_ccd_pt(Context& c, hipStream_t st, int pb) {
     Scene& s = c.sc;
     const LBVH& ft = c.sface_tree;
     const TreeView ftv{ft.n, ft.nodes.p, ft.wide.p};
-    hipLaunchKernelGGL(full_ccd_pt_kernel, dim3(blocks_for((size_t)s.Vs << pb, 64)), dim3(64), 0, st, s.Vs, s.sv_perm.p, s.sv.p,
+    hipLaunchKernelGGL(full_ccd_pt_kernel, dim3(blocks_for((size_t)s.Vs << pb, 16)), dim3(64), 0, st, s.Vs, s.sv_perm.p, s.sv.p,
                        s.faces.p, s.bt.p, s.x.p, s.dir.p, ftv, c.u64scratch.p, 1.0 - 0.8, scene_of_vertex(s), pb);
 }
 void launch_full_ccd_ee(Context& c, hipStream_t st, int pb) {
     Scene& s = c.sc;
     const LBVH& et = c.sedge_tree;
     const TreeView etv{et.n, et.nodes.p, et.wide.p, et.leafpos.p};
-    hipLaunchKernelGGL(full_ccd_ee_kernel, dim3(blocks_for((size_t)s.Es << pb, 64)), dim3(64), 0, st, s.Es, s.se_perm.p, s.se.p, s.bt.p,
-                       s.x.p, s.dir.p, etv, et.prim.p, c.u64scratch.p, 1.0 - 0.8, scene_of_vertex(s), pb);
+    hipLaunchKernelGGL(full_ccd_ee_kernel, dim3(blocks_for((size_t)s.Es << pb, 16)), dim3(64), 0, st, s.Es, s.se_perm.p, s.se.p, s.bt.p,
+                       s.x.p, s.dir.p, etv, c.u64scratch.p, 1.0 - 0.8, scene_of_vertex(s), pb);
 }
 
 // ---- autotuner ----------------------------------------------------------------------
@@ -301,13 +322,13 @@ __global__ void copy_slot(int S, int dst, int src, unsigned long long* sl) {
     if (k < S) sl[kSlots * k + dst] = sl[kSlots * k + src];
 }
 
-// Times every split of the two full-CCD walks and of the active set's two walks (1 to 16
+// Times every group size of the two full-CCD walks and of the active set's two walks (4 to 64
 // lanes per query) on the current positions and direction, three runs each after one warm-up, with HIP events on the
 // context's stream, and keeps the fastest for the context's later step bounds.  Each run
 // starts from the minimum the walk starts from in a step bound (slot 3 reseeded from the
 // swept step, slot 5, for the point-triangle walk and from the point-triangle result, slot
 // 4, for the edge-edge walk), so the pruning is the one a step bound sees.  Each walk's
-// result is a minimum over pairs, so every split gives the same step.
+// result is a minimum over pairs, so every group size gives the same step.
 int autotune(Context& c, TuneEntry* out, int max_out) {
     Scene& s = c.sc;
     const int S = s.S;
@@ -350,7 +371,7 @@ int autotune(Context& c, TuneEntry* out, int max_out) {
     // the active set's walks, on the static trees of the current positions (the set is built
     // once first; each walk writes only its hit counts and buffers, so runs repeat exactly)
     active_set_now(c);
-    size_active_walks(c, kTuneSplits - 1, kTuneSplits - 1);
+    size_active_walks(c);
     for (int k = 3; k <= 4; ++k) {
         const bool pt = k == 3;
         if (pt ? (s.Vs == 0 || c.face_tree.n <= 0) : (s.Es == 0 || c.edge_tree.n <= 0)) continue;
@@ -362,7 +383,7 @@ int autotune(Context& c, TuneEntry* out, int max_out) {
             float total = 0.f;
             for (int r = 0; r < 4; ++r) {
                 CIPC_HIP(hipEventRecord(e0, c.stream));
-                launch_active_walk(c, pt, false, pb);
+                launch_active_walks(c, pt, !pt, false, pb, pb, c.stream);
                 CIPC_HIP(hipEventRecord(e1, c.stream));
                 CIPC_HIP(hipEventSynchronize(e1));
                 float ms = 0.f;

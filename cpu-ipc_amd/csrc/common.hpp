@@ -143,17 +143,21 @@ struct alignas(64) Node {
     d3 hi;
     int right, pad;
 };
-// Four-wide record of an internal node: the boxes of its grandchildren (its children where
-// those are leaves), rounded outward to float, and what they are: the binary node index of
-// an internal node, -(primitive + 1) for a leaf, kNoChild for an empty slot.  One 128-byte
-// line per step of a wide walk; boxes that only touch after rounding are kept, so a wide
-// walk returns a superset that the caller confirms with the exact boxes.
+// Four-wide record of an internal node, one 128-byte line: its grandchildren (its children
+// where those are leaves), 32 bytes each so that four lanes test one record with two 16-byte
+// loads a lane: the box, rounded outward to float, and what it is: the binary node index of
+// an internal node, -(primitive + 1) for a leaf, kNoChild for an empty slot.  Boxes that only
+// touch after rounding are kept, so a wide walk returns a superset that the caller confirms
+// with the exact boxes.
 constexpr int kNoChild = 0x7fffffff;
+struct alignas(16) WideChild {
+    float lo[3];
+    int child;
+    float hi[3];
+    int last;    // last leaf position under the child
+};
 struct alignas(128) Node4 {
-    float lo[4][3];
-    float hi[4][3];
-    int child[4];
-    int pad[4];
+    WideChild c[4];
 };
 // Touching counts as overlapping (CPU IPC/LBVH.cpp:157-161); `q` is the querying box.
 __host__ __device__ inline bool overlaps(const Box& q, const Box& b, double gap) {

@@ -69,7 +69,7 @@ struct ActiveSetScratch {
     int capPT = 0, capEE = 0, capM = 0;
     // per point query, per edge query and per surface vertex (ground flag), in one array
     DBuf<int> cnt_all, off_all;
-    DBuf<int> cntpPT, cntpEE, bufPT, bufEE;
+    DBuf<int> bufPT, bufEE;
     DBuf<int> candUPT, candUEE, candPT, candEE, ownPT, ownEE, catPT, catEE;
     DBuf<int4> recPT, recEE;
     DBuf<int2> auxEE;
@@ -142,7 +142,7 @@ struct Context {
         long long captures = 0, replays = 0;
     } graph;
     unsigned long long topo_gen = 0;   // tree topologies built (broadphase.hip)
-    // tile choices of the autotuner (ccd.hip): lanes per query of the full-CCD walks (2^bits)
+    // tile choices of the autotuner (ccd.hip): lanes per query, 4 << bits, of the full-CCD walks
     // and of the active set's walks
     struct Tune {
         int ccd_pt_bits = 3, ccd_ee_bits = 3;
@@ -340,14 +340,28 @@ void step_bound_launch(Context& c, hipStream_t st);
 void step_bound_early(Context& c, hipStream_t st, bool ground = true);
 void step_bound_partial(Context& c, hipStream_t st);
 void step_bound_finish(Context& c, double* out);
-void size_active_walks(Context& c, int pt, int ee);
-void launch_active_walk(Context& c, bool pt, bool compact, int pb, hipStream_t st = nullptr);
+void size_active_walks(Context& c);
+void launch_active_walks(Context& c, bool pt, bool ee, bool compact, int pb, int eb, hipStream_t st);
+// A walk's lanes per query, 4 << bits, until the autotuner chooses: the largest bits up to 3
+// with queries << bits <= limit.  More lanes take fewer steps over a query, fewer lanes waste
+// less of a step on a short stack once the queries fill the chip; the limits split the sizes
+// timed (microseconds for bits 0..4, queries 600 to 172,000):
+//   active set, edges   2x11^3 cubes 26/17/15/10/12, 4x32^3 46/44/40/54/95, batch 82/79/88/131/234
+//   active set, points  2x11^3 29/14/10/9/9, 4x32^3 38/20/17/23/35, batch 30/23/29/46/79
+//   full CCD, edges     2x11^3 28/19/15/16/21, 4x32^3 53/52/71/115/200, batch 105/121/180/299/517
+//   full CCD, points    2x11^3 32/31/24/24/25, 4x32^3 38/38/56/75/110, batch 47/50/70/114/179
+constexpr int kWalkPoints = 1 << 17, kWalkEdges = 1 << 18, kCcdPoints = 1 << 16, kCcdEdges = 3 << 15;
+inline int walk_bits(int queries, int limit) {
+    int b = 0;
+    while (b < 3 && ((long long)queries << (b + 1)) <= limit) ++b;
+    return b;
+}
 void launch_full_ccd_pt(Context& c, hipStream_t st, int pb);
 void launch_full_ccd_ee(Context& c, hipStream_t st, int pb);
 // the autotuner: one entry per tuned kernel (0 full CCD point-triangle, 1 edge-edge, 3 the
 // active set's point-triangle walk, 4 its edge-edge walk), the mean ms of each candidate
 // split and the chosen one; returns the number of entries
-constexpr int kTuneSplits = 5;     // 1, 2, 4, 8 or 16 lanes per query
+constexpr int kTuneSplits = 5;     // 4, 8, 16, 32 or 64 lanes per query
 struct TuneEntry {
     int kernel = 0, chosen = 0, n = 0;
     double ms[8] = {};

@@ -278,15 +278,15 @@ int cipc_gpu_step_bound(cipc_gpu_context* ctx, double out[5]);
  * loops (ContactMechanics.cpp:3754-3867) with no launch shape to choose.  It times each
  * candidate split of the two full-CCD walks of the step bound (kernel 0 point-triangle,
  * 1 edge-edge) and of the active set's two walks (kernel 3 point-triangle, 4 edge-edge;
- * candidate c runs 2^c lanes per query, c = 0..4) on the context's current positions and
+ * candidate c runs 4 * 2^c lanes per query, c = 0..4) on the context's current positions and
  * direction (cipc_gpu_set_direction; a batch context times its whole batch), and keeps the
  * fastest for every later call of the context.  Every split returns the same results, bit
  * for bit: a full-CCD walk's result is a minimum over pairs, and the active set ranks its
  * hits by primitive.  entries (may be NULL) receives up to max_entries records (4 at most),
  * n_entries the number of tuned kernels.
  * cipc_gpu_set_tune sets a choice directly (an uploaded scene starts with the largest c,
- * at most 4, that keeps 2^c times the walk's query count (surface vertices or surface
- * edges) within 2^17 lanes); its
+ * at most 3, that keeps 2^c times the walk's query count (surface vertices or surface
+ * edges) within a limit per walk); its
  * kernel 2 switches the Newton iteration's single graph launch (cipc_gpu_newton_iteration,
  * cipc_gpu_batch_newton_iteration) off (choice 0: every stage launched on its own and timed)
  * or on (1); by default a batch context uses it and a single-scene context does not. */
