@@ -907,8 +907,8 @@ void enqueue_iteration(cipc_gpu_context* c, double kappa, bool energy, const Ite
     // energy on `aux`; then the CSR on the main stream.  Host enqueue time is close to half
     // the iteration's GPU time, so its order decides how long the main stream waits.
     if (t) CIPC_HIP(hipEventRecord(t->ev[0], c->stream));
-    CIPC_HIP(hipEventRecord(c->it_start, c->stream));
     contact_records_prepare(*c);
+    CIPC_HIP(hipEventRecord(c->it_start, c->stream));
     compute_active_set(*c, false);   // contact_assemble publishes the counts
     if (t) CIPC_HIP(hipEventRecord(t->ev[1], c->stream));
     CIPC_HIP(hipEventRecord(c->as_done, c->stream));
@@ -982,7 +982,8 @@ bool iteration_graph(cipc_gpu_context* c, double kappa, bool energy, hipEvent_t 
     // by default a batch goes as one graph launch and a single scene eagerly (measured no
     // faster as a graph: launching the graph's ~120 nodes costs the host what the launches do)
     const bool on = c->graph.mode < 0 ? c->sc.S > 1 : c->graph.mode == 1;
-    if (!on || !trees_refit_only(c) || c->capS == 0 || c->as.capPT == 0) return false;
+    // (an enqueue that was cut short has left the bucket counts for an eager one to clear)
+    if (!on || !trees_refit_only(c) || c->capS == 0 || c->as.capPT == 0 || c->bucket_cnt_clear == 0) return false;
     std::vector<unsigned char> key = iter_key(c, kappa, energy);
     if (!c->graph.exec || key != c->graph.key) {
         drop_graph(c);

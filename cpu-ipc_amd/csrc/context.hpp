@@ -196,35 +196,33 @@ struct Context {
     DBuf<int4> fverts;
 
     // contact contributions (fixed slots, invalid key = ~0ull)
-    DBuf<unsigned long long> ckey, ckey_sorted;
-    DBuf<int> cidx, cidx_sorted;
+    DBuf<unsigned long long> ckey;
     DBuf<double> cval;         // 9 per record
     DBuf<int> cdims;           // per contact: local Hessian dimension
     DBuf<int4> cverts;         // per contact: vertices (-1 past the last)
     DBuf<double> chess;        // per contact: 78 upper-triangle Hessian + 12 gradient entries (SoA)
     DBuf<int> gkey, gkey_sorted, gidx, gidx_sorted;
-    // vertex buckets that order the records (sparse.hip): counts and cursors, starts, entries
-    DBuf<int> bucket_cnt, bucket_start;
+    // vertex buckets that order the records (sparse.hip): counts and totals, starts, the list of
+    // those with records, each record's slot, entries
+    DBuf<int> bucket_cnt, bucket_start, bucket_list, bucket_slot;
     size_t bucket_cnt_clear = 0;        // leading entries of bucket_cnt known to be zero (left so by the last assembly)
     const int* bucket_cnt_ptr = nullptr;  // the buffer they are known zero in
-    DBuf<unsigned long long> bucket_entries;
+    DBuf<unsigned long long> bucket_entries, bucket_sorted;
     DBuf<double> gval;         // 3 per record
-    DBuf<int> run_start;       // start of each run of equal sorted contact block keys
-    DBuf<unsigned long long> ukey;  // unique contact block keys
+    DBuf<int> urow;            // unique contact blocks of each column, at its bucket's start
     DBuf<double> uval;
     DBuf<unsigned short> uflag;
-    int64_t n_ublocks = 0;
     DBuf<int> counters;        // small scratch integers
 
     // merged block pattern and output CSR
-    DBuf<int> mptr, mrow, mcol;
-    DBuf<int> pcnt, ppos;      // scalar runs of (merged block, column component) pairs
+    DBuf<int> mptr, mrow, mcol;   // mptr: V + 1 block column starts, then the scan's 3V + 1 scalar columns
+    DBuf<int> merge_cnt;
+    DBuf<int2> merge_src;         // (static, contact) block of each merged block of a column with contact blocks
     DBuf<double> mval;
-    DBuf<unsigned short> mflag;
     DBuf<int> outer, inner;
     DBuf<double> val, rhs;
     int64_t nnz = 0;
-    DBuf<int> coll;            // collision count of the last finalize_csr (device)
+    DBuf<int> coll;            // nonzeros and collision count of the last finalize_csr (device), the count's running sums
     bool nnz_pending = false;  // nnz and the collision count are in pin_nnz once the stream has been synchronised
     // pinned destinations of the asynchronous reads that one final synchronisation collects
     PinnedBuf<int> pin_nnz;
@@ -272,7 +270,7 @@ void build_tet_chunks(Context& c, const double* hx);
 void elastic_assemble(Context& c, hipStream_t st);
 void cloth_assemble(Context& c, hipStream_t st);
 // contact.hip
-// contact_records_prepare sizes the records (host only); friction_records_launch builds the
+// contact_records_prepare sizes the records and clears their counts; friction_records_launch builds the
 // lagged friction records on a stream; contact_assemble the barrier records (and, unless
 // friction_launched, prepares and launches the friction records itself on `aux`).
 void contact_records_prepare(Context& c);
@@ -280,6 +278,7 @@ void friction_records_launch(Context& c, hipStream_t st);
 void contact_assemble(Context& c, double kappa, bool friction_launched = false);
 // sparse.hip
 // count_collisions false: the caller launches collision_count_launch and publish_nnz itself
+void bucket_records_prepare(Context& c, size_t nb, size_t ng);
 void finalize_csr(Context& c, bool count_collisions = true);
 void collision_count_launch(Context& c, hipStream_t st);
 void publish_nnz(Context& c, hipStream_t st);

@@ -7,9 +7,10 @@
 // column-major lower storage (outer = column starts, inner = ascending rows), and the
 // right-hand side zeroed on non-free vertices.
 //
-// Pipeline: sort contact block records by (column vertex, row vertex), sum equal keys
-// in record order; merge them per block column with the static pattern; expand the
-// merged 3x3 blocks to scalar entries keeping exactly those that received a nonzero
+// Pipeline: contact records bucketed by block column (gradient records by vertex), each bucket
+// sorted and its equal blocks summed in record order by one wavefront; the merged block and
+// scalar entry counts of every column with the static pattern; one scan; one pass that writes
+// the merged 3x3 blocks and the CSR, with exactly the scalar entries that received a nonzero
 // contribution.
 #include "context.hpp"
 
@@ -52,7 +53,6 @@ void exclusive_scan_int(Context& c, const int* in, int* out, int n) {
     CIPC_HIP(hipcub::DeviceScan::ExclusiveSum(c.tmp.p, bytes, in, out, n, c.stream));
 }
 
-// --- contact block records: equal-key runs (heads from bucket_tails), their sums and nonzero masks -----
 // End of the run of `key` that starts at i in the sorted keys (galloping, then bisection), so
 // that the summation loop has known bounds and its loads are independent.
 template <typename K>
@@ -62,42 +62,6 @@ __device__ inline int run_end(const K* __restrict__ k, int n, int i, K key) {
     if (b > n) b = n;
     while (b - a > 1) { const int m = (a + b) >> 1; if (k[m] == key) a = m; else b = m; }
     return b;
-}
-// Start of every run, in run order (start[pos[i]] = i at each head), and one past the last
-// keyed record after the last run, so that run o is [start[o], start[o + 1]).
-__global__ void run_starts_u64(int n, const unsigned long long* __restrict__ k, const int* __restrict__ head,
-                               const int* __restrict__ pos, int* __restrict__ start) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i > n) return;
-    if (i < n && head[i]) start[pos[i]] = i;
-    const bool end = (i == n) ? (n == 0 || k[n - 1] != kNoKey) : (k[i] == kNoKey && (i == 0 || k[i - 1] != kNoKey));
-    if (end) start[pos[n]] = i;
-}
-// One thread per run (unique block): the records' 3x3 values summed in record order, entries
-// equal to zero skipped, and the mask of entries that received a nonzero value.
-__global__ void reduce_blocks(int n, const unsigned long long* __restrict__ k, const int* __restrict__ idx,
-                              const int* __restrict__ start, const int* __restrict__ pos, const double* __restrict__ val,
-                              unsigned long long* __restrict__ ukey, double* __restrict__ uval, unsigned short* __restrict__ uflag) {
-    const int o = blockIdx.x * blockDim.x + threadIdx.x;
-    if (o >= pos[n]) return;
-    const int i = start[o], e = start[o + 1];
-    const unsigned long long key = k[i];
-    double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    unsigned mask = 0;
-#pragma unroll 2
-    for (int j = i; j < e; ++j) {
-        const double* v = val + (size_t)9 * idx[j];
-#pragma unroll
-        for (int c = 0; c < 9; ++c) {
-            const bool nz = v[c] != 0.0;
-            acc[c] += nz ? v[c] : 0.0;   // exact: an accumulator starting at +0 never holds -0
-            mask |= nz ? (1u << c) : 0u;
-        }
-    }
-    ukey[o] = key;
-#pragma unroll
-    for (int c = 0; c < 9; ++c) uval[(size_t)9 * o + c] = acc[c];
-    uflag[o] = (unsigned short)mask;
 }
 // --- contact gradient records, summed per vertex in record order ------------------
 __global__ void add_gradient_records(int n, const int* __restrict__ k, const int* __restrict__ idx,
@@ -120,173 +84,187 @@ void add_gradient_records_into(Context& c, int n, const int* k, const int* idx, 
     hipLaunchKernelGGL(add_gradient_records, dim3(blocks_for(n, 256)), dim3(256), 0, c.stream, n, k, idx, val, c.sc.V, grad);
     CIPC_CHECK_LAUNCH();
 }
-// --- merge static and contact blocks per block column --------------------------------
-__device__ inline int lower_bound_u64(const unsigned long long* a, int n, unsigned long long key) {
-    int lo = 0, hi = n;
-    while (lo < hi) { const int m = (lo + hi) >> 1; if (a[m] < key) lo = m + 1; else hi = m; }
-    return lo;
-}
-__global__ void merge_count(int V, int kb, const int* __restrict__ scol, const int* __restrict__ srow,
-                            const unsigned long long* __restrict__ ukey, const int* __restrict__ nu_ptr, int* __restrict__ cnt) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b == 0) cnt[V] = 0;   // the scan's tail
-    if (b >= V) return;
-    const int nu = *nu_ptr;
-    int i = scol[b], ie = scol[b + 1];
-    int j = lower_bound_u64(ukey, nu, (unsigned long long)b << kb);
-    const int je = lower_bound_u64(ukey, nu, (unsigned long long)(b + 1) << kb);
-    int n = 0;
-    while (i < ie || j < je) {
-        const int ra = i < ie ? srow[i] : 0x7fffffff;
-        const int rb = j < je ? (int)(ukey[j] & ((1ull << kb) - 1)) : 0x7fffffff;
-        if (ra == rb) { ++i; ++j; } else if (ra < rb) ++i; else ++j;
-        ++n;
-    }
-    cnt[b] = n;
-}
-__global__ void merge_fill(int V, int kb, const int* __restrict__ scol, const int* __restrict__ srow, const double* __restrict__ sbv,
-                           const unsigned short* __restrict__ sbf, const unsigned long long* __restrict__ ukey,
-                           const double* __restrict__ uval, const unsigned short* __restrict__ uflag, const int* __restrict__ nu_ptr,
-                           const int* __restrict__ mptr, int* __restrict__ mrow, int* __restrict__ mcol, double* __restrict__ mval,
-                           unsigned short* __restrict__ mflag) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= V) return;
-    const int nu = *nu_ptr;
-    int i = scol[b], ie = scol[b + 1];
-    int j = lower_bound_u64(ukey, nu, (unsigned long long)b << kb);
-    const int je = lower_bound_u64(ukey, nu, (unsigned long long)(b + 1) << kb);
-    int o = mptr[b];
-    while (i < ie || j < je) {
-        const int ra = i < ie ? srow[i] : 0x7fffffff;
-        const int rb = j < je ? (int)(ukey[j] & ((1ull << kb) - 1)) : 0x7fffffff;
-        double v[9];
-        unsigned f = 0;
-        if (ra <= rb) {
-#pragma unroll
-            for (int e = 0; e < 9; ++e) v[e] = sbv[(size_t)9 * i + e];
-            f = sbf[i];
-        } else {
-#pragma unroll
-            for (int e = 0; e < 9; ++e) v[e] = 0.0;
-        }
-        if (rb <= ra) {
-#pragma unroll
-            for (int e = 0; e < 9; ++e) v[e] += uval[(size_t)9 * j + e];
-            f |= uflag[j];
-        }
-        mrow[o] = ra < rb ? ra : rb;
-        mcol[o] = b;
-#pragma unroll
-        for (int e = 0; e < 9; ++e) mval[(size_t)9 * o + e] = v[e];
-        mflag[o] = (unsigned short)f;
-        ++o;
-        if (ra == rb) { ++i; ++j; } else if (ra < rb) ++i; else ++j;
-    }
-}
-// --- scalar expansion: DOF column j = 3b + cc ------------------------------------------
-// Scalar CSR.  Scalar column 3b + cc lists, for each merged block k of block column b in
-// row order, the rows r of k with a nonzero flag at (r, cc) (r >= cc on the diagonal block).
-// Each (block, component) pair therefore owns a contiguous run of the column; the pairs
-// are laid out (b, cc, k) so one exclusive scan of their counts gives every run's start,
-// and the column starts are the starts of each column's first run.
-__device__ inline int pair_index(const int* __restrict__ mptr, int b, int cc, int k) {
-    const int m0 = mptr[b];
-    return 3 * m0 + cc * (mptr[b + 1] - m0) + (k - m0);
-}
-__global__ void pair_count(const int* __restrict__ nm_ptr, const int* __restrict__ mptr, const int* __restrict__ mrow,
-                           const int* __restrict__ mcol, const unsigned short* __restrict__ mflag, int* __restrict__ cnt) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nm = *nm_ptr;
-    if (t > 3 * nm) return;
-    if (t == 3 * nm) { cnt[t] = 0; return; }
-    const int k = t / 3, cc = t % 3;
-    const int b = mcol[k];
-    const unsigned f = mflag[k];
-    const int r0 = (mrow[k] == b) ? cc : 0;
-    int n = 0;
-    for (int r = r0; r < 3; ++r) n += (f >> (3 * r + cc)) & 1u;
-    cnt[pair_index(mptr, b, cc, k)] = n;
-}
-// outer[j]: the column starts; the last one, the nonzero count, also into nnz_out
-__device__ inline void column_starts(int j, int V, const int* __restrict__ mptr, const int* __restrict__ ppos,
-                                     const int* __restrict__ nm_ptr, int* __restrict__ outer, int* __restrict__ nnz_out) {
-    if (j > 3 * V) return;
-    if (j == 3 * V) {
-        const int nnz = ppos[3 * *nm_ptr];
-        outer[j] = nnz;
-        *nnz_out = nnz;
-        return;
-    }
-    const int b = j / 3, cc = j % 3;
-    outer[j] = ppos[pair_index(mptr, b, cc, mptr[b])];
-}
-__device__ inline void pair_fill(int t, const int* __restrict__ nm_ptr, const int* __restrict__ mptr, const int* __restrict__ mrow,
-                                 const int* __restrict__ mcol, const double* __restrict__ mval, const unsigned short* __restrict__ mflag,
-                                 const int* __restrict__ ppos, int* __restrict__ inner, double* __restrict__ val) {
-    if (t >= 3 * *nm_ptr) return;
-    const int k = t / 3, cc = t % 3;
-    const int b = mcol[k], a = mrow[k];
-    const unsigned f = mflag[k];
-    int o = ppos[pair_index(mptr, b, cc, k)];
-    for (int r = (a == b) ? cc : 0; r < 3; ++r) {
-        if ((f >> (3 * r + cc)) & 1u) {
-            inner[o] = 3 * a + r;
-            val[o] = mval[(size_t)9 * k + 3 * r + cc];
-            ++o;
-        }
-    }
-}
-__device__ inline void masked_rhs(int i, int V, const int* __restrict__ bt, const double* __restrict__ grad, double* __restrict__ rhs) {
-    if (i >= 3 * V) return;
-    rhs[i] = is_free(bt[i / 3]) ? grad[i] : 0.0;
-}
-// The CSR's last three steps in one launch (they read what earlier launches wrote and write
-// disjoint arrays): work-groups [0, bC) the column starts, the next bP the entries of the
-// merged blocks, the rest the right-hand side.
-struct CsrFinish {
-    int V, bC, bP;
-    const int *mptr, *ppos, *nm_ptr, *mrow, *mcol, *bt;
-    const double *mval, *grad;
-    const unsigned short* mflag;
-    int *outer, *nnz_out, *inner;
+// --- static and contact blocks merged per block column; the scalar CSR -------------------
+// A block's flags: bit 3r + c set where entry (r, c) received a nonzero contribution.  Scalar
+// column 3b + c lists, for each merged block of block column b in row order, the rows r of the
+// block with a flag at (r, c) (r >= c on the diagonal block).
+constexpr unsigned kLowerFlags = 0x1d9u;   // (r, c) with r >= c
+__device__ inline unsigned csr_flags(unsigned f, bool diagonal) { return diagonal ? f & kLowerFlags : f; }
+
+struct Merge {
+    int V, nblocks, nb;
+    const int *scol, *srow;              // static blocks
+    const double* sbv;
+    const unsigned short* sbf;
+    int* ucnt;                           // unique contact blocks of column b: ucnt[2b], at ustart[2b]
+    const int *ustart, *urow;
+    const double* uval;
+    const unsigned short* uflag;
+    const int* mstart;
+    int2* src;                           // (static, contact) block or -1 of each merged block, at mstart
+    int *count, *off;                    // merged blocks per column (V + 1), then entries per scalar column (3V + 1)
+    int* totals;
+    const int* bt;
+    const double* grad;
+    int *mrow, *mcol;
+    double* mval;
+    int *outer, *inner, *nnz_out;
     double *val, *rhs;
 };
-__global__ void csr_finish(CsrFinish a) {
-    int b = blockIdx.x;
-    if (b < a.bC) {
-        column_starts(b * blockDim.x + threadIdx.x, a.V, a.mptr, a.ppos, a.nm_ptr, a.outer, a.nnz_out);
-        return;
+// One thread per block column: how many blocks and scalar entries it has, and, where it has
+// contact blocks, which two each merged block comes from.  Only flags and rows are read: the
+// values wait for csr_fill, which knows every start.
+__global__ void merge_count(Merge a) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    int* entries = a.count + a.V + 1;
+    if (b == 0) {   // the scan's tails
+        a.count[a.V] = 0;
+        entries[3 * a.V] = 0;
     }
-    b -= a.bC;
-    if (b < a.bP) {
-        pair_fill(b * blockDim.x + threadIdx.x, a.nm_ptr, a.mptr, a.mrow, a.mcol, a.mval, a.mflag, a.ppos, a.inner, a.val);
-        return;
+    if (b >= a.V) return;
+    const int nu = a.ucnt[2 * b], ie = a.scol[b + 1];
+    int i = a.scol[b], n = 0, e0 = 0, e1 = 0, e2 = 0;
+    auto add = [&](unsigned f) {
+        ++n;
+        e0 += __popc(f & 0x49u);
+        e1 += __popc(f & 0x92u);
+        e2 += __popc(f & 0x124u);
+    };
+    if (nu == 0) {
+        for (; i < ie; ++i) add(csr_flags(a.sbf[i], a.srow[i] == b));
+    } else {
+        int j = a.ustart[2 * b];
+        const int je = j + nu;
+        int2* src = a.src + a.mstart[b];
+        while (i < ie || j < je) {
+            const int ra = i < ie ? a.srow[i] : 0x7fffffff, rb = j < je ? a.urow[j] : 0x7fffffff;
+            const bool st = ra <= rb, co = rb <= ra;
+            src[n] = make_int2(st ? i : -1, co ? j : -1);
+            add(csr_flags((st ? a.sbf[i] : 0u) | (co ? a.uflag[j] : 0u), min(ra, rb) == b));
+            i += st ? 1 : 0;
+            j += co ? 1 : 0;
+        }
     }
-    b -= a.bP;
-    masked_rhs(b * blockDim.x + threadIdx.x, a.V, a.bt, a.grad, a.rhs);
+    a.count[b] = n;
+    entries[3 * b] = e0; entries[3 * b + 1] = e1; entries[3 * b + 2] = e2;
+}
+// The merged blocks, the CSR and the right-hand side in one pass: kFillLanes lanes per block
+// column, a merged block each (most columns have 7 or 8).  A lane's scalar entries follow those
+// of the lanes before it, which ballots count.  It is bound by its stores (a 72-byte block is
+// written twice, once with its indices): 94 us on four 32^3 cubes (1.1 million blocks), where a
+// thread per column, counts per block and component, their scan and a fill took 205.
+constexpr int kFillLanes = 8;
+__global__ __launch_bounds__(256) void csr_fill(Merge a) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int b = t / kFillLanes, l = t % kFillLanes, g0 = (threadIdx.x & 63) - l;
+    const int base = a.off[a.V + 1];   // the entries' counts follow the blocks' in the scan
+    const int* ent = a.off + a.V + 1;
+    if (t == 0) {
+        const int nnz = ent[3 * a.V] - base;
+        a.outer[3 * a.V] = nnz;
+        *a.nnz_out = nnz;
+        a.totals[0] = a.totals[1] = a.totals[2] = a.totals[3] = 0;   // the buckets' totals for the next assembly
+    }
+    const bool on = b < a.V;
+    int m0 = 0, nm = 0, nu = 0, s0 = 0;
+    int pos[3] = {0, 0, 0};
+    const int2* src = nullptr;
+    if (on) {
+        m0 = a.off[b];
+        nm = a.off[b + 1] - m0;
+        nu = a.ucnt[2 * b];
+        s0 = a.scol[b];
+        if (nu) src = a.src + a.mstart[b];
+        for (int c = 0; c < 3; ++c) pos[c] = ent[3 * b + c] - base;
+        if (l < 3) {
+            a.outer[3 * b + l] = l == 0 ? pos[0] : l == 1 ? pos[1] : pos[2];
+            a.rhs[3 * (size_t)b + l] = is_free(a.bt[b]) ? a.grad[3 * (size_t)b + l] : 0.0;
+        }
+    }
+    const unsigned long long before = (1ull << l) - 1, lanes = (1ull << kFillLanes) - 1;
+    for (int p0 = 0; __any(p0 < nm); p0 += kFillLanes) {
+        const int p = p0 + l;
+        const bool has = p < nm;
+        int i = -1, j = -1, row = 0;
+        unsigned f = 0;
+        double v[9];
+        if (has) {
+            if (nu) {
+                const int2 x = src[p];
+                i = x.x; j = x.y;
+            } else {
+                i = s0 + p;
+            }
+            row = i >= 0 ? a.srow[i] : a.urow[j];
+            if (i >= 0) {
+                f = a.sbf[i];
+#pragma unroll
+                for (int e = 0; e < 9; ++e) v[e] = a.sbv[(size_t)9 * i + e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 9; ++e) v[e] = 0.0;
+            }
+            if (j >= 0) {
+                f |= a.uflag[j];
+#pragma unroll
+                for (int e = 0; e < 9; ++e) v[e] += a.uval[(size_t)9 * j + e];
+            }
+            const size_t o = (size_t)m0 + p;
+            a.mrow[o] = row;
+            a.mcol[o] = b;
+#pragma unroll
+            for (int e = 0; e < 9; ++e) a.mval[9 * o + e] = v[e];
+            f = csr_flags(f, row == b);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            int o = pos[c], all = 0;
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                const unsigned long long m = (__ballot((f >> (3 * r + c)) & 1u) >> g0) & lanes;
+                o += __popcll(m & before);
+                all += __popcll(m);
+            }
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+                if ((f >> (3 * r + c)) & 1u) {
+                    a.inner[o] = 3 * row + r;
+                    a.val[o] = v[3 * r + c];
+                    ++o;
+                }
+            pos[c] += all;
+        }
+    }
+    if (on && l == 0 && nu) a.ucnt[2 * b] = 0;   // for the next assembly's bucket counts
 }
 
 // Collision count as compute_g_dpt returns it (ContactMechanics.cpp:2970-3032): the
-// multiplicity of a point-point / point-edge entry, one for every other Self_ActiveSet
-// entry.  One work-group, integer sums: the result does not depend on the order.
-// out[0] = the CSR's nonzeros (nnz_dev), out[1] = the collision count: read by the host together.
-// *out: compute_g_dpt's count over Self_ActiveSet (one per entry, the multiplicity for a
-// point-point or point-edge map entry)
-__global__ void collision_count(const int* __restrict__ n_dev, const int4* __restrict__ set, int* __restrict__ out) {
-    __shared__ long long sh[256];
-    long long acc = 0;
+// multiplicity of a point-point / point-edge entry, one for every other Self_ActiveSet entry.
+// out[1] = the count, out[0] = the CSR's nonzeros (csr_fill): read by the host together.  The
+// work-groups add their sums to out[2], and the last of them (out[3] counts) publishes and
+// clears both.  (One work-group over the whole set took 336 us on a folded 128^2 cloth's 105,000
+// entries, 9 now.)
+constexpr int kCountGroups = 128;
+__global__ __launch_bounds__(256) void collision_count(const int* __restrict__ n_dev, const int4* __restrict__ set, int* out) {
+    __shared__ int sh[4];
+    int acc = 0;
     const int n = *n_dev;
-    for (int i = threadIdx.x; i < n; i += 256) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         const int4 e = set[i];
-        acc += (e.x < 0 && (e.z < 0 || e.w < 0)) ? -(long long)e.w : 1ll;
+        acc += (e.x < 0 && (e.z < 0 || e.w < 0)) ? -e.w : 1;
     }
-    sh[threadIdx.x] = acc;
+    for (int w = 32; w > 0; w >>= 1) acc += __shfl_xor(acc, w);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-        __syncthreads();
+    if (threadIdx.x != 0) return;
+    acc = sh[0] + sh[1] + sh[2] + sh[3];
+    atomicAdd(out + 2, acc);
+    __threadfence();
+    if (atomicAdd(out + 3, 1) == (int)gridDim.x - 1) {
+        __threadfence();
+        out[1] = atomicExch(out + 2, 0);
+        atomicExch(out + 3, 0);
     }
-    if (threadIdx.x == 0) *out = (int)sh[0];
 }
 
 __global__ void zero_ints(int* __restrict__ p, int n) {
@@ -294,171 +272,240 @@ __global__ void zero_ints(int* __restrict__ p, int n) {
     if (i < n) p[i] = 0;
 }
 
-
-// --- contact records bucketed by vertex: the order of a stable sort by key ----------
-// The block records are bucketed by block column (the key's high field) and the gradient
-// records by vertex: counts per bucket (integer atomics, order-free), one scan of both count
-// arrays for the bucket starts, a scatter (atomic slot within the bucket), and one wavefront
-// per bucket that orders it by (row, record) / record and writes the keys and record indices
-// as a stable sort by key over all records would (records without a key last).  This
-// replaces a global radix sort: every bucket is small, and the whole takes five launches.
-__global__ void bucket_count(int n, const unsigned long long* __restrict__ bkey, int kb, int ng, const int* __restrict__ gkey, int V,
-                             int* __restrict__ bcnt, int* __restrict__ gcnt) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        const unsigned long long k = bkey[i];
-        if (k != kNoKey) atomicAdd(bcnt + (int)(k >> kb), 1);
-    }
-    if (i < ng) {
-        const int v = gkey[i];
-        if (v >= 0 && v < V) atomicAdd(gcnt + v, 1);
-    }
-}
-// bucket entries in one array: block records as (row, record) at [0, blocks), gradient
-// records as their record index after them, where the joint scan's starts place them
-__global__ void bucket_scatter(int n, const unsigned long long* __restrict__ bkey, int kb, const int* __restrict__ bstart,
-                               int* __restrict__ bfill, int ng, const int* __restrict__ gkey, int V, const int* __restrict__ gstart,
-                               int* __restrict__ gfill, unsigned long long* __restrict__ entries) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        const unsigned long long k = bkey[i];
-        if (k != kNoKey) {
-            const int b = (int)(k >> kb);
-            const unsigned row = (unsigned)(k & ((1ull << kb) - 1));
-            entries[bstart[b] + atomicAdd(bfill + b, 1)] = ((unsigned long long)row << 32) | (unsigned)i;
-        }
-    }
-    if (i < ng) {
-        const int v = gkey[i];
-        if (v >= 0 && v < V) entries[gstart[v] + atomicAdd(gfill + v, 1)] = (unsigned long long)(unsigned)i;
-    }
-}
-constexpr int kBucketWaves = 2;
-constexpr int kBucketLds = 2048;
-__device__ inline unsigned long long shfl_xor_u64(unsigned long long v, int m) {
-    const unsigned lo = __shfl_xor((unsigned)v, m), hi = __shfl_xor((unsigned)(v >> 32), m);
-    return ((unsigned long long)hi << 32) | lo;
-}
-__device__ inline void bucket_wave_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-// Output of entry t of bucket bk (sorted entry e): a block record's key and index, or a
-// gradient record's vertex and index.
-struct BucketOut {
-    int V, kb, gbase;
-    unsigned long long* bkey;
-    int* bidx;
-    int* gkey;
-    int* gidx;
-    __device__ void put(int bk, int pos, unsigned long long e) const {
-        if (bk < V) {
-            bkey[pos] = ((unsigned long long)(unsigned)bk << kb) | (e >> 32);
-            bidx[pos] = (int)(e & 0xffffffffu);
-        } else {
-            gkey[pos - gbase] = bk - V - 1;
-            gidx[pos - gbase] = (int)(e & 0xffffffffu);
-        }
-    }
+// --- contact records bucketed by vertex and summed --------------------------------------
+// Bucket 2v holds the block records of block column v, bucket 2v + 1 the gradient records of
+// vertex v.  The kernels that write the records count them (Records in contact.hip: one atomic
+// per contact and vertex gives the records of both buckets their slots).  Then a start per
+// bucket that has records, from running totals (where a bucket lies decides nothing), and the
+// list of those buckets; the scatter; and one work-group per listed bucket that puts its records
+// in the order of a stable sort by key and sums them in that order.  Most vertices of a body are
+// in no contact, so nothing is launched per vertex but the pass over the counts.
+struct Buckets {
+    int V, kb, nb, ng;
+    const unsigned long long* bkey;
+    const int *gkey, *slot;           // slot: nb block records', then ng gradient records'
+    int *cnt, *start, *list;          // 2V
+    int* mstart;                      // V: room for a column's merged blocks
+    const int* scol;
+    int* totals;                      // listed buckets, block entries, gradient entries, merged blocks of columns with entries
+    unsigned long long *entries, *sorted;   // nb + ng: (row, record) of blocks, then records of gradients
+    const double *cval, *gval;
+    int* urow;                        // at a column's start: its unique blocks
+    double* uval;
+    unsigned short* uflag;
+    double* grad;
 };
-// Bucket bk = [starts[bk], starts[bk + 1]) of the 2V + 1 buckets, k > 1 entries, sorted by
-// one wavefront: up to 64 entries in registers (bitonic network over the lanes), up to
-// kBucketLds in LDS (bitonic network, the wave ordering its own LDS accesses between steps),
-// longer buckets by one lane in place.
-__device__ inline void sort_bucket(int bk, int s0, int k, int lane, unsigned long long* __restrict__ a,
-                                   unsigned long long* __restrict__ keys, const BucketOut& out) {
-    if (k <= 64) {
-        unsigned long long v = lane < k ? keys[s0 + lane] : ~0ull;
-#pragma unroll
-        for (int size = 2; size <= 64; size <<= 1)
-#pragma unroll
-            for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                const unsigned long long o = shfl_xor_u64(v, stride);
-                const bool keep_min = ((lane & stride) == 0) == ((lane & size) == 0);
-                v = keep_min ? (o < v ? o : v) : (o > v ? o : v);
-            }
-        if (lane < k) out.put(bk, s0 + lane, v);
-        return;
+__device__ inline int wave_prefix(int v, int& total) {
+    const int lane = threadIdx.x & 63;
+    int x = v;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(x, d);
+        if (lane >= d) x += y;
     }
-    if (k <= kBucketLds) {
-        int P = 128;
-        while (P < k) P <<= 1;
-        for (int i = lane; i < P; i += 64) a[i] = i < k ? keys[s0 + i] : ~0ull;
-        bucket_wave_order();
-        for (int size = 2; size <= P; size <<= 1)
-            for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                for (int t = lane; t < (P >> 1); t += 64) {
-                    const int i = 2 * stride * (t / stride) + (t % stride), j = i + stride;
-                    const unsigned long long x = a[i], y = a[j];
-                    const bool asc = (i & size) == 0;
-                    if ((x > y) == asc) { a[i] = y; a[j] = x; }
-                }
-                bucket_wave_order();
-            }
-        for (int i = lane; i < k; i += 64) out.put(bk, s0 + i, a[i]);
-        bucket_wave_order();   // the LDS is the next bucket's
-        return;
+    total = __shfl(x, 63);
+    return x - v;
+}
+// One atomic per total and work-group: they all fall on the same words (one per wavefront took
+// 47 us on a batch of 40 scenes with 380,000 buckets, one per work-group takes 8).
+constexpr int kStartsBlock = 1024;
+__global__ __launch_bounds__(kStartsBlock) void bucket_starts(Buckets a) {
+    __shared__ int part[kStartsBlock / 64][4], base[4];
+    const int bk = blockIdx.x * kStartsBlock + threadIdx.x, w = threadIdx.x >> 6;
+    const int k = bk < 2 * a.V ? a.cnt[bk] : 0;
+    const bool column = k > 0 && (bk & 1) == 0;
+    const int want[4] = {k > 0 ? 1 : 0, column ? k : 0, column ? 0 : k, column ? k + a.scol[(bk >> 1) + 1] - a.scol[bk >> 1] : 0};
+    int at[4], sum;
+    for (int c = 0; c < 4; ++c) {
+        at[c] = wave_prefix(want[c], sum);
+        if ((threadIdx.x & 63) == 0) part[w][c] = sum;
     }
-    if (lane == 0) {
-        for (int i = s0 + 1; i < s0 + k; ++i) {
-            const unsigned long long x = keys[i];
-            int j = i - 1;
-            while (j >= s0 && keys[j] > x) { keys[j + 1] = keys[j]; --j; }
-            keys[j + 1] = x;
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        sum = 0;
+        for (int i = 0; i < kStartsBlock / 64; ++i) {
+            const int x = part[i][threadIdx.x];
+            part[i][threadIdx.x] = sum;
+            sum += x;
         }
-        for (int i = s0; i < s0 + k; ++i) out.put(bk, i, keys[i]);
+        base[threadIdx.x] = sum ? atomicAdd(a.totals + threadIdx.x, sum) : 0;
     }
+    __syncthreads();
+    if (k == 0) return;
+    for (int c = 0; c < 4; ++c) at[c] += base[c] + part[w][c];
+    a.list[at[0]] = bk;
+    a.start[bk] = column ? at[1] : at[2];
+    if (column) a.mstart[bk >> 1] = at[3];
 }
-// Each wavefront takes bpw consecutive buckets (1 or 64): a lane writes its bucket's entry
-// when it has one, and the wave sorts the longer ones together, one after the other.  64
-// when the record slots are fewer than the buckets (most buckets then have none or one: a
-// batch of scenes with few contacts), else 1, so that long buckets (vertices in many
-// contacts, often neighbours) are not sorted one after the other by one wavefront.
-__global__ __launch_bounds__(64 * kBucketWaves) void bucket_sort(int nbk, int bpw, const int* __restrict__ starts,
-                                                                 unsigned long long* __restrict__ keys, BucketOut out) {
-    __shared__ unsigned long long sh[kBucketWaves][kBucketLds];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int bk0 = (blockIdx.x * kBucketWaves + w) * bpw;
-    if (bk0 >= nbk) return;   // the whole wavefront: no block-wide barrier follows
-    out.gbase = starts[out.V + 1];   // the gradient entries follow the block entries
-    const int bk = bk0 + lane;
-    int s0 = 0, k = 0;
-    if (lane < bpw && bk < nbk) {
-        s0 = starts[bk];
-        k = starts[bk + 1] - s0;
-    }
-    if (k == 1) out.put(bk, s0, keys[s0]);
-    unsigned long long big = __ballot(k > 1);
-    while (big) {
-        const int l = __ffsll((long long)big) - 1;
-        big &= big - 1;
-        sort_bucket(bk0 + l, __shfl(s0, l), __shfl(k, l), lane, sh[w], keys, out);
-    }
-}
-// Records without a key, after the keyed ones: block keys kNoKey, gradient keys past every vertex.
-// After the bucket sort, in one launch: the unkeyed records after the keyed ones (as a stable
-// sort leaves them), the run heads of the sorted block keys (head[nb] = 0: the scan's total
-// is the run count), and the bucket counters cleared for the next assembly (nothing after
-// the bucket scatter reads them).  Keys past the keyed ones are the sentinel whether or not
-// this launch has written them yet.
-__global__ void bucket_tails(int nb, int ng, const int* __restrict__ starts, int V, unsigned long long* __restrict__ bkey,
-                             int* __restrict__ bidx, int* __restrict__ gkey, int* __restrict__ gidx, int* __restrict__ head,
-                             int* __restrict__ counters, int ncounters) {
+__global__ void bucket_scatter(Buckets a) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int tb = starts[V], tg = starts[2 * V + 1] - starts[V + 1];
-    if (i < nb) {
-        const unsigned long long k = i < tb ? bkey[i] : kNoKey;
-        if (i >= tb) { bkey[i] = kNoKey; bidx[i] = i; }
-        const unsigned long long kp = i == 0 ? 0ull : (i - 1 < tb ? bkey[i - 1] : kNoKey);
-        head[i] = (k != kNoKey && (i == 0 || k != kp)) ? 1 : 0;
-    } else if (i == nb) {
-        head[nb] = 0;
+    if (i < a.nb) {
+        const unsigned long long k = a.bkey[i];
+        if (k != kNoKey)
+            a.entries[a.start[2 * (int)(k >> a.kb)] + a.slot[i]] = ((k & ((1ull << a.kb) - 1)) << 32) | (unsigned)i;
     }
-    if (i >= tg && i < ng) { gkey[i] = 0x7fffffff; gidx[i] = i; }
-    if (i < ncounters) counters[i] = 0;
+    if (i < a.ng) {
+        const int v = a.gkey[i];
+        if (v < a.V) a.entries[(size_t)a.nb + a.start[2 * v + 1] + a.slot[a.nb + i]] = (unsigned)i;
+    }
+}
+// One work-group of two wavefronts per listed bucket (vertices in contact have 20 to 300 block
+// records).  Every entry is placed by its rank, the number of smaller ones (all are distinct;
+// a bitonic network by one wavefront took longer than everything else here): kBucketLds entries
+// in LDS at a time, the result in LDS if they all fit.  Then kSumBlock entries at a time: their
+// values into LDS, all loads in flight at once and neighbouring lanes reading neighbouring
+// values, and a column's runs of equal rows, a lane per entry of the 3x3 block, zero entries
+// skipped, with the flags of entries that received a nonzero value; a vertex's gradient by a lane
+// per component.  Bound by the latency of one bucket's chain while the buckets are few.
+// From the records to the sums: 5 + 5 + 63 us on four 20^3 cubes in contact and 25 us on two
+// 11^3, where two scans, a sort by one wavefront, a thread per run and a thread per gradient
+// took 223 and 82.
+constexpr int kSumBlock = 128, kBucketLds = 512;
+struct BucketLds {
+    union {
+        unsigned long long e[kBucketLds];
+        double val[kSumBlock * 9];
+    };
+    unsigned long long sorted[kBucketLds];
+    int start[kSumBlock + 1], heads[kSumBlock / 64];
+};
+// sorted[rank] of the bucket's entries [i0, i0 + N kSumBlock)
+template <int N>
+__device__ inline void place_entries(const unsigned long long* __restrict__ entries, int i0, int k, BucketLds& sh,
+                                     unsigned long long* sorted) {
+    const int t = threadIdx.x;
+    unsigned long long v[N];
+    int rank[N];
+    for (int c = 0; c < N; ++c) {
+        const int i = i0 + kSumBlock * c + t;
+        v[c] = i < k ? entries[i] : 0ull;
+        rank[c] = 0;
+    }
+    for (int j0 = 0; j0 < k; j0 += kBucketLds) {
+        const int m = min(kBucketLds, k - j0);
+        __syncthreads();
+        for (int j = t; j < m; j += kSumBlock) sh.e[j] = entries[j0 + j];
+        __syncthreads();
+#pragma unroll 4
+        for (int j = 0; j < m; ++j) {
+            const unsigned long long x = sh.e[j];
+#pragma unroll
+            for (int c = 0; c < N; ++c) rank[c] += x < v[c] ? 1 : 0;
+        }
+    }
+    for (int c = 0; c < N; ++c)
+        if (i0 + kSumBlock * c + t < k) sorted[rank[c]] = v[c];
+}
+__device__ inline void place_bucket(const unsigned long long* __restrict__ entries, int k, BucketLds& sh, unsigned long long* sorted) {
+    for (int i0 = 0; i0 < k; i0 += 4 * kSumBlock) {
+        if (k - i0 <= kSumBlock) place_entries<1>(entries, i0, k, sh, sorted);
+        else if (k - i0 <= 2 * kSumBlock) place_entries<2>(entries, i0, k, sh, sorted);
+        else place_entries<4>(entries, i0, k, sh, sorted);
+    }
+    __syncthreads();
+}
+__device__ inline void sum_gradients(const Buckets& a, int v, int k, const unsigned long long* e, BucketLds& sh) {
+    const int t = threadIdx.x;
+    double* g = a.grad + 3 * (size_t)v + t;
+    double sum = t < 3 ? *g : 0.0;
+    for (int i0 = 0; i0 < k; i0 += kSumBlock) {
+        const int m = min(kSumBlock, k - i0);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const int q = t + kSumBlock * c;
+            if (q < 3 * m) sh.val[q] = a.gval[(size_t)3 * (unsigned)e[i0 + q / 3] + q % 3];
+        }
+        __syncthreads();
+        if (t < 3)
+#pragma unroll 8
+            for (int j = 0; j < m; ++j) sum += sh.val[3 * j + t];
+        __syncthreads();
+    }
+    if (t < 3) *g = sum;
+}
+// The sums of a column's runs at s0, and how many there are.
+__device__ inline int sum_column(const Buckets& a, int s0, int k, const unsigned long long* e, BucketLds& sh) {
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, l = lane / 9, c = lane - 9 * l;
+    int u = 0;
+    for (int i0 = 0; i0 < k; i0 += kSumBlock) {
+        const int m = min(kSumBlock, k - i0), i = i0 + t;
+#pragma unroll
+        for (int x = 0; x < 9; ++x) {
+            const int q = t + kSumBlock * x;
+            if (q < 9 * m) sh.val[q] = a.cval[(size_t)9 * (unsigned)e[i0 + q / 9] + q % 9];
+        }
+        const bool head = i < k && (i == 0 || (e[i] >> 32) != (e[i - 1] >> 32));
+        const unsigned long long heads = __ballot(head);
+        if (lane == 0) sh.heads[w] = __popcll(heads);
+        const int cont = i0 > 0 && (e[i0] >> 32) == (e[i0 - 1] >> 32) ? 1 : 0;    // the last chunk's last run goes on
+        __syncthreads();
+        const int nr = sh.heads[0] + sh.heads[1] + cont, r0 = s0 + u - cont;
+        const int o = cont + (w ? sh.heads[0] : 0) + __popcll(heads & ((1ull << lane) - 1));
+        if (head) {
+            sh.start[o] = t;
+            a.urow[r0 + o] = (int)(e[i] >> 32);
+        }
+        if (t == 0) {
+            if (cont) sh.start[0] = 0;
+            sh.start[nr] = m;
+        }
+        __syncthreads();
+        for (int q = 7 * w; q < nr; q += 14) {
+            const int r = q + l;
+            const bool on = l < 7 && r < nr;
+            double sum = 0.0;
+            bool any = false;
+            if (on) {
+                if (r == 0 && cont) {
+                    sum = a.uval[(size_t)9 * r0 + c];
+                    any = (a.uflag[r0] >> c) & 1;
+                }
+                const int end = sh.start[r + 1];
+                for (int j = sh.start[r]; j < end; ++j) {
+                    const double x = sh.val[9 * j + c];
+                    const bool nz = x != 0.0;
+                    sum += nz ? x : 0.0;   // exact: an accumulator starting at +0 never holds -0
+                    any |= nz;
+                }
+                a.uval[(size_t)9 * (r0 + r) + c] = sum;
+            }
+            const unsigned long long f = __ballot(on && any);
+            if (on && c == 0) a.uflag[r0 + r] = (unsigned short)((f >> (9 * l)) & 0x1ffu);
+        }
+        u += nr - cont;
+        __syncthreads();   // the LDS is the next chunk's, whose first run may read the last sum
+    }
+    return u;
+}
+__global__ __launch_bounds__(kSumBlock) void bucket_sums(Buckets a) {
+    __shared__ BucketLds sh;
+    const int n = a.totals[0];
+    for (int t = blockIdx.x; t < n; t += gridDim.x) {
+        const int bk = a.list[t], k = a.cnt[bk], s0 = a.start[bk];
+        const size_t at = (size_t)(bk & 1 ? a.nb : 0) + s0;
+        unsigned long long* sorted = k <= kBucketLds ? sh.sorted : a.sorted + at;
+        int u = 0;   // a gradient bucket's count is cleared for the next assembly
+        place_bucket(a.entries + at, k, sh, sorted);
+        if (bk & 1) sum_gradients(a, bk >> 1, k, sorted, sh);
+        else u = sum_column(a, s0, k, sorted, sh);
+        if (threadIdx.x == 0) a.cnt[bk] = u;
+        __syncthreads();   // the LDS is the next bucket's
+    }
 }
 
+// Room for nb block and ng gradient records, and their buckets' counts cleared where the last
+// assembly is not known to have left them so (a new buffer, a larger scene, an enqueue cut
+// short).  Before the launches that write the records.
+void bucket_records_prepare(Context& c, size_t nb, size_t ng) {
+    const size_t ncnt = 2 * (size_t)c.sc.V + 4;   // counts, then the totals
+    c.bucket_cnt.resize(ncnt);
+    c.bucket_slot.resize(nb + ng + 1);
+    if (c.bucket_cnt_clear < ncnt || c.bucket_cnt_ptr != c.bucket_cnt.p) {
+        hipLaunchKernelGGL(zero_ints, dim3(blocks_for(ncnt, 256)), dim3(256), 0, c.stream, c.bucket_cnt.p, (int)ncnt);
+        CIPC_CHECK_LAUNCH();
+    }
+    c.bucket_cnt_clear = 0;
+    c.bucket_cnt_ptr = c.bucket_cnt.p;
+}
 // The nonzero and collision counts (c.coll) to pinned memory, for the host's next
 // synchronisation.
 void publish_nnz(Context& c, hipStream_t st) {
@@ -468,126 +515,58 @@ void publish_nnz(Context& c, hipStream_t st) {
 }
 // The collision count of the assembly's set (c.coll[1]), on stream st.
 void collision_count_launch(Context& c, hipStream_t st) {
-    c.coll.resize(2);
-    hipLaunchKernelGGL(collision_count, dim3(1), dim3(256), 0, st, c.dcnt.p + kDcSelf, c.self_set.p, c.coll.p + 1);
+    if (c.coll.n < 4) {
+        c.coll.resize(4);
+        hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, st, c.coll.p + 2, 2);   // from then on each count leaves its sums cleared
+    }
+    hipLaunchKernelGGL(collision_count, dim3(kCountGroups), dim3(256), 0, st, c.dcnt.p + kDcSelf, c.self_set.p, c.coll.p);
     CIPC_CHECK_LAUNCH();
 }
 
 void finalize_csr(Context& c, bool count_collisions) {
     Scene& s = c.sc;
     const int V = s.V;
-    // contact block records
-    const int nb = (int)c.ckey.n;
-    c.ckey_sorted.resize(std::max(nb, 1)); c.cidx_sorted.resize(std::max(nb, 1));
-    c.iscratch2.resize(std::max<size_t>((size_t)3 * V + 1, (size_t)nb + 2));
-    c.counters.resize(4);
-    c.ukey.resize(std::max(nb, 1)); c.uval.resize((size_t)9 * std::max(nb, 1)); c.uflag.resize(std::max(nb, 1));
-    int* head = c.iscratch2.p;
-    int* pos = nullptr;
-    c.iscratch.resize((size_t)std::max(nb, 1) + 1);
-    pos = c.iscratch.p;
-    const int ng = (int)c.gkey.n;
-    // the records of both kinds in key order, bucketed by vertex (counts of the block columns
-    // and of the gradient vertices adjacent: one scan)
-    {
-        c.bucket_cnt.resize(4 * ((size_t)V + 1));
-        int* bcnt = c.bucket_cnt.p;
-        int* gcnt = bcnt + (V + 1);
-        int* bfill = gcnt + (V + 1);
-        int* gfill = bfill + (V + 1);
-        c.bucket_start.resize(2 * ((size_t)V + 1));
-        int* bstart = c.bucket_start.p;
-        int* gstart = bstart + (V + 1);
-        c.bucket_entries.resize((size_t)nb + ng + 1);
-        c.gkey_sorted.resize(std::max(ng, 1)); c.gidx_sorted.resize(std::max(ng, 1));
-        // the counters are left cleared by the previous assembly's bucket_tails; cleared here
-        // when that is not known (a new buffer, a larger scene, an enqueue cut short)
-        const size_t ncnt = 4 * ((size_t)V + 1);
-        if (c.bucket_cnt_clear < ncnt || c.bucket_cnt_ptr != bcnt)
-            hipLaunchKernelGGL(zero_ints, dim3(blocks_for(ncnt, 256)), dim3(256), 0, c.stream, bcnt, (int)ncnt);
-        c.bucket_cnt_clear = 0;
-        c.bucket_cnt_ptr = bcnt;
-        const int nmax = std::max(nb, ng);
-        if (nmax > 0)
-            hipLaunchKernelGGL(bucket_count, dim3(blocks_for(nmax, 256)), dim3(256), 0, c.stream, nb, c.ckey.p, s.kb, ng, c.gkey.p, V,
-                               bcnt, gcnt);
-        CIPC_CHECK_LAUNCH();
-        exclusive_scan_int(c, bcnt, bstart, 2 * (V + 1));
-        if (nmax > 0) {
-            hipLaunchKernelGGL(bucket_scatter, dim3(blocks_for(nmax, 256)), dim3(256), 0, c.stream, nb, c.ckey.p, s.kb, bstart, bfill,
-                               ng, c.gkey.p, V, gstart, gfill, c.bucket_entries.p);
-            const BucketOut bo{V, s.kb, 0, c.ckey_sorted.p, c.cidx_sorted.p, c.gkey_sorted.p, c.gidx_sorted.p};
-            const int bpw = (size_t)nb + ng < 2 * (size_t)V + 1 ? 64 : 1;
-            hipLaunchKernelGGL(bucket_sort, dim3(blocks_for(2 * V + 1, kBucketWaves * bpw)), dim3(64 * kBucketWaves), 0,
-                               c.stream, 2 * V + 1, bpw, bstart, c.bucket_entries.p, bo);
-            const size_t nt = std::max<size_t>(std::max<size_t>((size_t)nb + 1, (size_t)ng), ncnt);
-            hipLaunchKernelGGL(bucket_tails, dim3(blocks_for(nt, 256)), dim3(256), 0, c.stream, nb, ng, bstart, V, c.ckey_sorted.p,
-                               c.cidx_sorted.p, c.gkey_sorted.p, c.gidx_sorted.p, head, bcnt, (int)ncnt);
-        }
-        CIPC_CHECK_LAUNCH();
-        c.bucket_cnt_clear = ncnt;   // by bucket_tails, or never touched (no records)
-    }
-    if (nb > 0) {
-        exclusive_scan_int(c, head, pos, nb + 1);
-        c.run_start.resize((size_t)nb + 2);
-        hipLaunchKernelGGL(run_starts_u64, dim3(blocks_for(nb + 1, 256)), dim3(256), 0, c.stream, nb, c.ckey_sorted.p, head, pos,
-                           c.run_start.p);
-        hipLaunchKernelGGL(reduce_blocks, dim3(blocks_for(nb, 256)), dim3(256), 0, c.stream, nb, c.ckey_sorted.p,
-                           c.cidx_sorted.p, c.run_start.p, pos, c.cval.p, c.ukey.p, c.uval.p, c.uflag.p);
-        CIPC_CHECK_LAUNCH();
-    } else {
-        hipLaunchKernelGGL(zero_ints, dim3(1), dim3(64), 0, c.stream, c.counters.p, 1);
+    const int nb = (int)c.ckey.n, ng = (int)c.gkey.n;
+    if (count_collisions) collision_count_launch(c, c.stream);   // (else the caller has, on a stream of its own)
+    // the contact records' sums: unique blocks per column, gradients into c.grad
+    Buckets k;
+    k.V = V; k.kb = s.kb; k.nb = nb; k.ng = ng; k.bkey = c.ckey.p; k.gkey = c.gkey.p;
+    c.bucket_start.resize(3 * (size_t)V); c.bucket_list.resize(2 * (size_t)V);
+    c.bucket_entries.resize((size_t)nb + ng + 1); c.bucket_sorted.resize((size_t)nb + ng + 1);
+    c.urow.resize((size_t)nb + 1); c.uval.resize((size_t)9 * (nb + 1)); c.uflag.resize((size_t)nb + 1);
+    k.cnt = c.bucket_cnt.p; k.totals = k.cnt + 2 * V; k.start = c.bucket_start.p; k.list = c.bucket_list.p; k.slot = c.bucket_slot.p;
+    k.mstart = k.start + 2 * V; k.scol = c.sp.col_ptr.p;
+    k.entries = c.bucket_entries.p; k.sorted = c.bucket_sorted.p; k.cval = c.cval.p; k.gval = c.gval.p;
+    k.urow = c.urow.p; k.uval = c.uval.p; k.uflag = c.uflag.p; k.grad = c.grad.p;
+    const int nmax = std::max(nb, ng);
+    if (nmax > 0) {
+        hipLaunchKernelGGL(bucket_starts, dim3(blocks_for(2 * (size_t)V, kStartsBlock)), dim3(kStartsBlock), 0, c.stream, k);
+        hipLaunchKernelGGL(bucket_scatter, dim3(blocks_for(nmax, 256)), dim3(256), 0, c.stream, k);
+        // no more work-groups than fit the chip at once
+        const int groups = (int)std::min<size_t>(std::min<size_t>(2 * (size_t)V, (size_t)nb + ng), 256 * 10);
+        hipLaunchKernelGGL(bucket_sums, dim3(groups), dim3(kSumBlock), 0, c.stream, k);
         CIPC_CHECK_LAUNCH();
     }
-    // the number of unique contact blocks: the run scan's total (zero without records)
-    const int* nu_ptr = nb > 0 ? pos + nb : c.counters.p;
-    // contact gradient records
-    if (ng > 0) {
-        hipLaunchKernelGGL(add_gradient_records, dim3(blocks_for(ng, 256)), dim3(256), 0, c.stream, ng, c.gkey_sorted.p,
-                           c.gidx_sorted.p, c.gval.p, V, c.grad.p);
-        CIPC_CHECK_LAUNCH();
-    }
-    // merged block pattern, sized by its bound (static blocks + unique contact blocks <= records)
-    c.mptr.resize((size_t)V + 1);
-    DBuf<int>& cnt = c.iscratch2;
-    hipLaunchKernelGGL(merge_count, dim3(blocks_for(V, 256)), dim3(256), 0, c.stream, V, s.kb, c.sp.col_ptr.p, c.sp.row.p, c.ukey.p,
-                       nu_ptr, cnt.p);
+    // merged blocks and scalar entries, sized by their bounds (static blocks + contact records,
+    // 9 entries each)
+    const size_t mcap = (size_t)c.sp.nblocks + (size_t)nb + 1, nscan = 4 * (size_t)V + 2;
+    c.merge_src.resize(mcap); c.merge_cnt.resize(nscan); c.mptr.resize(nscan);
+    c.mrow.resize(mcap); c.mcol.resize(mcap); c.mval.resize(9 * mcap);
+    c.outer.resize((size_t)3 * V + 1); c.inner.resize(9 * mcap); c.val.resize(9 * mcap); c.rhs.resize((size_t)3 * V);
+    Merge a;
+    a.V = V; a.nblocks = (int)c.sp.nblocks; a.nb = nb; a.scol = c.sp.col_ptr.p; a.srow = c.sp.row.p; a.sbv = c.sbv.p; a.sbf = c.sbf.p;
+    a.ucnt = k.cnt; a.ustart = k.start; a.mstart = k.mstart; a.urow = k.urow; a.uval = k.uval; a.uflag = k.uflag; a.src = c.merge_src.p;
+    a.count = c.merge_cnt.p; a.off = c.mptr.p; a.totals = k.totals; a.bt = s.bt.p; a.grad = c.grad.p;
+    a.mrow = c.mrow.p; a.mcol = c.mcol.p; a.mval = c.mval.p; a.outer = c.outer.p; a.inner = c.inner.p; a.nnz_out = c.coll.p;
+    a.val = c.val.p; a.rhs = c.rhs.p;
+    hipLaunchKernelGGL(merge_count, dim3(blocks_for(V, 256)), dim3(256), 0, c.stream, a);
     CIPC_CHECK_LAUNCH();
-    exclusive_scan_int(c, cnt.p, c.mptr.p, V + 1);
-    const size_t mcap = (size_t)c.sp.nblocks + (size_t)nb + 1;
-    c.mrow.resize(mcap); c.mcol.resize(mcap); c.mval.resize(9 * mcap); c.mflag.resize(mcap);
-    hipLaunchKernelGGL(merge_fill, dim3(blocks_for(V, 256)), dim3(256), 0, c.stream, V, s.kb, c.sp.col_ptr.p, c.sp.row.p, c.sbv.p,
-                       c.sbf.p, c.ukey.p, c.uval.p, c.uflag.p, nu_ptr, c.mptr.p, c.mrow.p, c.mcol.p, c.mval.p, c.mflag.p);
+    exclusive_scan_int(c, a.count, a.off, (int)nscan);   // mptr: the first V + 1
+    hipLaunchKernelGGL(csr_fill, dim3(blocks_for((size_t)V * kFillLanes, 256)), dim3(256), 0, c.stream, a);
     CIPC_CHECK_LAUNCH();
-    // scalar CSR: (block, component) counts -> one scan -> column starts and runs
-    const int* nm_ptr = c.mptr.p + V;
-    c.pcnt.resize(3 * mcap + 1); c.ppos.resize(3 * mcap + 1);
-    hipLaunchKernelGGL(pair_count, dim3(blocks_for(3 * mcap + 1, 256)), dim3(256), 0, c.stream, nm_ptr, c.mptr.p, c.mrow.p, c.mcol.p,
-                       c.mflag.p, c.pcnt.p);
-    CIPC_CHECK_LAUNCH();
-    // the scan covers the bound; entries past 3 nm + 1 are never read
-    exclusive_scan_int(c, c.pcnt.p, c.ppos.p, (int)(3 * mcap + 1));
-    c.outer.resize((size_t)3 * V + 1);
-    c.coll.resize(2);
-    c.inner.resize(9 * mcap); c.val.resize(9 * mcap);
-    c.rhs.resize((size_t)3 * V);
-    {
-        CsrFinish a;
-        a.V = V; a.bC = (int)blocks_for(3 * V + 1, 256); a.bP = (int)blocks_for(3 * mcap, 256);
-        a.mptr = c.mptr.p; a.ppos = c.ppos.p; a.nm_ptr = nm_ptr; a.mrow = c.mrow.p; a.mcol = c.mcol.p; a.bt = s.bt.p;
-        a.mval = c.mval.p; a.grad = c.grad.p; a.mflag = c.mflag.p; a.outer = c.outer.p; a.nnz_out = c.coll.p;
-        a.inner = c.inner.p; a.val = c.val.p; a.rhs = c.rhs.p;
-        hipLaunchKernelGGL(csr_finish, dim3(a.bC + a.bP + (int)blocks_for(3 * V, 256)), dim3(256), 0, c.stream, a);
-        CIPC_CHECK_LAUNCH();
-    }
-    // the counts are read with the caller's next synchronisation (the collision count is
-    // launched here, or by the caller on a stream of its own before it publishes them); the
-    // entries are sized by their bound (9 per merged block)
-    if (count_collisions) {
-        collision_count_launch(c, c.stream);
-        publish_nnz(c, c.stream);
-    }
-    CIPC_CHECK_LAUNCH();
+    c.bucket_cnt_clear = c.bucket_cnt.n;
+    // the counts are read with the caller's next synchronisation (or the caller publishes them)
+    if (count_collisions) publish_nnz(c, c.stream);
 }
 
 }  // namespace cipc
