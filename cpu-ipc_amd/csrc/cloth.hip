@@ -116,16 +116,31 @@ __global__ __launch_bounds__(256) void bend_quad_kernel(int Nb, int e0, const in
     }
 }
 
-// One thread per hinge: E = D w dtheta^2 / 2, dtheta = remainder(theta - rest, 2 pi);
+// Hinge: E = D w dtheta^2 / 2, dtheta = remainder(theta - rest, 2 pi);
 // g = D w dtheta grad theta, H = makePD(D w (grad grad^T + dtheta Hess theta)), both times
 // dt^2 (HingeBending.cpp:79-106; IPCSolver.cpp:238-267).  The angle is translation-invariant,
 // so the projection runs on the translation-free subspace like the contact blocks.
-template <typename HT>
-__global__ __launch_bounds__(64) void bend_hinge_kernel(int Nb, int e0, const int4* __restrict__ bv, const double* __restrict__ x,
-                                                        const double* __restrict__ rest, const double* __restrict__ weight,
-                                                        double plate, double dt2, const int* __restrict__ slot_h,
-                                                        const int* __restrict__ slot_g, HT* __restrict__ stagH,
-                                                        double* __restrict__ stagG) {
+// Hs: the packed upper triangle before the projection.
+__device__ inline void hinge_block(const d3* q, const double* g, double s, double df, double* Hs) {
+    M3x B[10];
+    hinge_angle_hess(q, B);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = a; b < 4; ++b)
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int j = (a == b ? i : 0); j < 3; ++j) {
+                    const int r = 3 * a + i, c = 3 * b + j;
+                    Hs[Sym<12>::ix(r, c)] = s * (g[r] * g[c] + df * B[ub_index(a, b)].m[i][j]);
+                }
+}
+// One thread per hinge: gradient records, and the block into Hs (packed, SoA).
+__global__ __launch_bounds__(64) void hinge_local_kernel(int Nb, int e0, const int4* __restrict__ bv, const double* __restrict__ x,
+                                                         const double* __restrict__ rest, const double* __restrict__ weight,
+                                                         double plate, const int* __restrict__ slot_g, double* __restrict__ Hs,
+                                                         double* __restrict__ stagG) {
     const int h = blockIdx.x * blockDim.x + threadIdx.x;
     if (h >= Nb) return;
     const int4 id = bv[h];
@@ -141,35 +156,34 @@ __global__ __launch_bounds__(64) void bend_hinge_kernel(int Nb, int e0, const in
 #pragma unroll
     for (int a = 0; a < 4; ++a)
         st3(stagG, slot_g[4 * e + a], d3{s * df * g[3 * a], s * df * g[3 * a + 1], s * df * g[3 * a + 2]});
-    double Hs[78];
-    {
-        M3x B[10];
-        hinge_angle_hess(q, B);
+    double A[78];
+    hinge_block(q, g, s, df, A);
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int b = a; b < 4; ++b)
-#pragma unroll
-                for (int i = 0; i < 3; ++i)
-#pragma unroll
-                    for (int j = (a == b ? i : 0); j < 3; ++j) {
-                        const int r = 3 * a + i, c = 3 * b + j;
-                        Hs[Sym<12>::ix(r, c)] = s * (g[r] * g[c] + df * B[ub_index(a, b)].m[i][j]);
-                    }
-    }
-    project_contact<4>([&](int k) -> double& { return Hs[k]; });
-#pragma unroll
-    for (int lb = 0; lb < 10; ++lb) {
-        const int j = slot_h[10 * e + lb];
+    for (int k = 0; k < 78; ++k) Hs[(size_t)k * Nb + h] = A[k];
+}
+// Projection and Hessian records, 16 lanes per hinge (project_contact_row).  One thread per
+// hinge for all of it, 124 us for the 5,000 hinges of a 41^2 cloth, was as long as one thread's
+// projection; now 11 + 65.
+template <typename HT>
+__global__ __launch_bounds__(64) void hinge_project_kernel(int Nb, int e0, const int4* __restrict__ bv, double dt2,
+                                                           const int* __restrict__ slot_h, const double* __restrict__ Hs,
+                                                           HT* __restrict__ stagH) {
+    __shared__ double A[4][78], lds[4][12][9];
+    const int grp = threadIdx.x >> 4, lane = threadIdx.x & 15, h0 = 4 * blockIdx.x, h = h0 + grp, e = e0 + h;
+    for (int t = threadIdx.x; t < 4 * 78; t += 64)
+        if (h0 + t % 4 < Nb) A[t % 4][t / 4] = Hs[(size_t)(t / 4) * Nb + h0 + t % 4];
+    row_order();
+    project_contact_row(h < Nb, [&](int k) -> double& { return A[grp][k]; }, lds[grp]);
+    row_order();
+    if (h >= Nb) return;
+    const int4 id = bv[h];
+    for (int t = lane; t < 90; t += 16) {
+        const int lb = t / 9, k = t - 9 * lb, j = slot_h[10 * e + lb];
         if (j < 0) continue;
         const int a = lb_a(lb), b = lb_b(lb);
-        const bool tr = vid[a] < vid[b];
-        HT* o = stagH + (size_t)9 * j;
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int kk = 0; kk < 3; ++kk)
-                o[3 * i + kk] = (HT)(dt2 * (tr ? Hs[Sym<12>::ix(3 * a + kk, 3 * b + i)] : Hs[Sym<12>::ix(3 * a + i, 3 * b + kk)]));
+        const bool tr = (a == 0 ? id.x : a == 1 ? id.y : a == 2 ? id.z : id.w) < (b == 0 ? id.x : b == 1 ? id.y : b == 2 ? id.z : id.w);
+        const int r = tr ? k % 3 : k / 3, c = tr ? k / 3 : k % 3;
+        stagH[(size_t)9 * j + k] = (HT)(dt2 * A[grp][Sym<12>::ix(3 * a + r, 3 * b + c)]);
     }
 }
 
@@ -186,9 +200,13 @@ static void cloth_assemble_t(Context& c, hipStream_t st, HT* stagH) {
         if (s.bmode == 0)
             hipLaunchKernelGGL(bend_quad_kernel<HT>, dim3(blocks_for(s.Nb, 256)), dim3(256), 0, st, s.Nb, s.T + s.Tr, s.bverts.p, s.x.p,
                                s.bq.p, s.plate, dt2, c.sp.slot_h.p, c.sp.slot_g.p, stagH, c.stagG.p);
-        else
-            hipLaunchKernelGGL(bend_hinge_kernel<HT>, dim3(blocks_for(s.Nb, 64)), dim3(64), 0, st, s.Nb, s.T + s.Tr, s.bverts.p, s.x.p,
-                               s.brest.p, s.bweight.p, s.plate, dt2, c.sp.slot_h.p, c.sp.slot_g.p, stagH, c.stagG.p);
+        else {
+            c.hingeH.resize((size_t)78 * s.Nb);
+            hipLaunchKernelGGL(hinge_local_kernel, dim3(blocks_for(s.Nb, 64)), dim3(64), 0, st, s.Nb, s.T + s.Tr, s.bverts.p, s.x.p,
+                               s.brest.p, s.bweight.p, s.plate, c.sp.slot_g.p, c.hingeH.p, c.stagG.p);
+            hipLaunchKernelGGL(hinge_project_kernel<HT>, dim3(blocks_for(s.Nb, 4)), dim3(64), 0, st, s.Nb, s.T + s.Tr, s.bverts.p, dt2,
+                               c.sp.slot_h.p, c.hingeH.p, stagH);
+        }
         CIPC_CHECK_LAUNCH();
     }
 }
@@ -263,31 +281,24 @@ __global__ void bw_eval_kernel(int n, const double* __restrict__ F, double st, d
 __global__ __launch_bounds__(64) void hinge_eval_kernel(int n, const double* __restrict__ pts, const double* __restrict__ rest,
                                                         const double* __restrict__ weight, double plate, double* __restrict__ G,
                                                         double* __restrict__ H, double* __restrict__ E) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    d3 q[4];
-    for (int a = 0; a < 4; ++a) q[a] = ld3(pts, 4 * t + a);
-    double g[12];
-    const double th = hinge_angle_grad(q, g);
-    const double df = remainder(th - rest[t], 6.28318530717958647692);
-    const double s = plate * weight[t];
-    for (int i = 0; i < 12; ++i) G[12 * t + i] = s * df * g[i];
-    double Hs[78];
-    {
-        M3x B[10];
-        hinge_angle_hess(q, B);
-        for (int a = 0; a < 4; ++a)
-            for (int b = a; b < 4; ++b)
-                for (int i = 0; i < 3; ++i)
-                    for (int j = (a == b ? i : 0); j < 3; ++j) {
-                        const int r = 3 * a + i, c = 3 * b + j;
-                        Hs[Sym<12>::ix(r, c)] = s * (g[r] * g[c] + df * B[ub_index(a, b)].m[i][j]);
-                    }
+    __shared__ double Hs[4][78], lds[4][12][9];
+    const int grp = threadIdx.x >> 4, t = 4 * blockIdx.x + grp;
+    if (t < n && (threadIdx.x & 15) == 0) {
+        d3 q[4];
+        for (int a = 0; a < 4; ++a) q[a] = ld3(pts, 4 * t + a);
+        double g[12];
+        const double th = hinge_angle_grad(q, g);
+        const double df = remainder(th - rest[t], 6.28318530717958647692);
+        const double s = plate * weight[t];
+        for (int i = 0; i < 12; ++i) G[12 * t + i] = s * df * g[i];
+        hinge_block(q, g, s, df, Hs[grp]);
+        E[t] = 0.5 * plate * weight[t] * df * df;
     }
-    project_contact<4>([&](int k) -> double& { return Hs[k]; });
-    for (int r = 0; r < 12; ++r)
-        for (int c = 0; c < 12; ++c) H[144 * t + 12 * r + c] = Hs[Sym<12>::ix(r, c)];
-    E[t] = 0.5 * plate * weight[t] * df * df;
+    row_order();
+    project_contact_row(t < n, [&](int k) -> double& { return Hs[grp][k]; }, lds[grp]);
+    row_order();
+    if (t < n)
+        for (int k = threadIdx.x & 15; k < 144; k += 16) H[144 * t + k] = Hs[grp][Sym<12>::ix(k / 12, k % 12)];
 }
 
 }  // namespace cipc
@@ -320,7 +331,7 @@ extern "C" int cipc_gpu_eval_hinge_impl(int n, const double* pts, const double* 
     CIPC_HIP(hipMemcpy(dp.p, pts, sizeof(double) * 12 * n, hipMemcpyHostToDevice));
     CIPC_HIP(hipMemcpy(dr.p, rest, sizeof(double) * n, hipMemcpyHostToDevice));
     CIPC_HIP(hipMemcpy(dw.p, weight, sizeof(double) * n, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(hinge_eval_kernel, dim3(blocks_for(n, 64)), dim3(64), 0, 0, n, dp.p, dr.p, dw.p, plate, dg.p, dH.p, de.p);
+    hipLaunchKernelGGL(hinge_eval_kernel, dim3(blocks_for(n, 4)), dim3(64), 0, 0, n, dp.p, dr.p, dw.p, plate, dg.p, dH.p, de.p);
     CIPC_CHECK_LAUNCH();
     CIPC_HIP(hipMemcpy(g, dg.p, sizeof(double) * 12 * n, hipMemcpyDeviceToHost));
     CIPC_HIP(hipMemcpy(H, dH.p, sizeof(double) * 144 * n, hipMemcpyDeviceToHost));

@@ -58,10 +58,10 @@ __device__ inline void dist_gh(int type, const double* q, double* g, double* H) 
     }
 }
 
-// Kernel 1: local Hessian (upper triangle, SoA) and local gradient of every contact, in
-// two launches over the contact range [0, n_self + n_ee):
-//   contact_self_kernel, c < n_self: Self_ActiveSet entry, compute_H_dpt / compute_g_dpt
-//   contact_ee_kernel, otherwise   : Self_EE_ActiveSet entry, compute_H_dee / compute_g_dee
+// Kernel 1: local Hessian (upper triangle, SoA) and local gradient of every contact of the
+// range [0, n_self + n_ee):
+//   self_contact, c < n_self: Self_ActiveSet entry, compute_H_dpt / compute_g_dpt
+//   ee_contact, otherwise   : Self_EE_ActiveSet entry, compute_H_dee / compute_g_dee
 // The self form is instantiated per distance type, so that its arrays have indices fixed at
 // compile time and stay in registers.
 template <int Type>
@@ -98,10 +98,9 @@ __device__ inline int record_contacts(const int* __restrict__ dc, int& ns) {
 __global__ void contact_totals(int capS, int* __restrict__ dc) {
     if (blockIdx.x == 0 && threadIdx.x == 0) dc[kDcContactOver] = dc[kDcSelf] + dc[kDcMol] > capS ? 1 : 0;
 }
-__global__ __launch_bounds__(64) void contact_self_kernel(const int* __restrict__ dc, int n, const int4* __restrict__ self_set,
-                                                          const double* __restrict__ x, double hhat, Kap kap, double* __restrict__ Hs,
-                                                          double* __restrict__ Gs, int4* __restrict__ verts, int* __restrict__ dims) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ inline void self_contact(int c, const int* __restrict__ dc, int n, const int4* __restrict__ self_set,
+                                    const double* __restrict__ x, double hhat, Kap kap, double* __restrict__ Hs,
+                                    double* __restrict__ Gs, int4* __restrict__ verts, int* __restrict__ dims) {
     int n_self;
     record_contacts(dc, n_self);
     if (c >= n_self) return;
@@ -118,88 +117,128 @@ __global__ __launch_bounds__(64) void contact_self_kernel(const int* __restrict_
     verts[c] = make_int4(v[0], v[1], type >= 1 ? v[2] : -1, type >= 2 ? v[3] : -1);
     dims[c] = 3 * nv_of(type);
 }
-__global__ __launch_bounds__(64) void contact_ee_kernel(
-    const int* __restrict__ dc, int n, const int4* __restrict__ ee_set,
-    const int2* __restrict__ ee_ie, const int2* __restrict__ se, const double* __restrict__ x,
-    const double* __restrict__ vrest, double hhat, Kap kap, double* __restrict__ Hs, double* __restrict__ Gs,
-    int4* __restrict__ verts, int* __restrict__ dims) {
+// A mollified edge-edge contact whose distance is of type Type, as 12 x 12 over the edges' ends
+// (indMap of ContactMechanics.cpp:3627-3685).  All indices are fixed at compile time: where the
+// distance's vertices lie among the ends is selected, not indexed (arrays indexed by it lived in
+// scratch, and 876 contacts took 78 us; with the 13,209 others in the same launch 33 now).
+template <int Type>
+__device__ inline void ee_local(int c, int n, const int (&v)[4], const int (&e4)[4], const double* __restrict__ x,
+                                const double* __restrict__ vrest, double hhat, double kappa, double* __restrict__ Hs,
+                                double* __restrict__ Gs) {
+    constexpr int nvd = Type == 0 ? 2 : (Type == 1 ? 3 : 4), Nd = 3 * nvd;
+    d3 p[4], pe[4];
+    double qd[12], qe[12];
+#pragma unroll
+    for (int k = 0; k < nvd; ++k) { p[k] = ld3(x, v[k]); qd[3 * k] = p[k].x; qd[3 * k + 1] = p[k].y; qd[3 * k + 2] = p[k].z; }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { pe[k] = ld3(x, e4[k]); qe[3 * k] = pe[k].x; qe[3 * k + 1] = pe[k].y; qe[3 * k + 2] = pe[k].z; }
+    const double d = self_value(Type, p);
+    const double b = barrier_b(d, hhat), gb = barrier_g(d, hhat), hb = barrier_h(d, hhat);
+    const double ex = eps_x_of(ld3(vrest, e4[0]), ld3(vrest, e4[1]), ld3(vrest, e4[2]), ld3(vrest, e4[3]));
+    const double cr = ee_cross_sqn(pe[0], pe[1], pe[2], pe[3]);
+    const double mol = mol_e(cr, ex);
+    double H[144], gl[12], gd[12];
+    dist_gh(Type, qd, gl, H);
+    // the distance's vertex at end k: -1 for none (the last match, as the reference's loop leaves it)
+    int at[4] = {0, 1, 2, 3};
+    if (Type != 3) {
+        int map[3] = {0, 1, 2};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const bool m0 = v[0] == e4[k], m1 = !m0 && v[1] == e4[k], m2 = !m0 && !m1 && nvd == 3 && v[2] == e4[k];
+            map[0] = m0 ? k : map[0];
+            map[1] = m1 ? k : map[1];
+            map[2] = m2 ? k : map[2];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            at[k] = -1;
+#pragma unroll
+            for (int a = 0; a < nvd; ++a) at[k] = map[a < 3 ? a : 0] == k ? a : at[k];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            if (Type == 3) { gd[3 * k + r] = gl[3 * k + r]; continue; }
+            double g = 0.0;
+#pragma unroll
+            for (int a = 0; a < nvd; ++a) g = at[k] == a ? gl[3 * a + r] : g;
+            gd[3 * k + r] = g;
+        }
+    // mollifier gradient and Hessian of the cross norm
+    double gc[12], Hc[144];
+    ee_cross_gh(qe, gc, Hc);
+    double ge[12], qg = 0.0, qH = 0.0;
+    const bool act = cr < ex;
+    if (act) {
+        const double oe = 1.0 / ex;
+        qg = 2.0 * oe * (-oe * cr + 1.0);
+        qH = -2.0 / (ex * ex);
+    }
+#pragma unroll
+    for (int k = 0; k < 12; ++k) ge[k] = act ? gc[k] * qg : 0.0;
+    const double kgb = kappa * gb, kb = kappa * b, keh = kappa * mol * hb, keg = kappa * mol * gb;
+    int idx = 0;
+#pragma unroll
+    for (int r = 0; r < 12; ++r)
+#pragma unroll
+        for (int s = r; s < 12; ++s) {
+            double hd = 0.0;   // embedded distance Hessian entry
+            if (Type == 3) {
+                hd = H[r * 12 + s];
+            } else {
+#pragma unroll
+                for (int a = 0; a < nvd; ++a)
+#pragma unroll
+                    for (int e = 0; e < nvd; ++e)
+                        hd = at[r / 3] == a && at[s / 3] == e ? H[(3 * a + r % 3) * Nd + 3 * e + s % 3] : hd;
+            }
+            const double eH = act ? Hc[r * 12 + s] * qg + (qH * gc[r]) * gc[s] : 0.0;
+            const double kgg = (kgb * gd[r]) * ge[s];
+            const double kggT = (kgb * gd[s]) * ge[r];
+            Hs[(size_t)(idx++) * n + c] = kgg + kggT + kb * eH + (keh * gd[r]) * gd[s] + keg * hd;
+        }
+    const double gsc = kappa * (gb * mol);
+#pragma unroll
+    for (int k = 0; k < 12; ++k) Gs[(size_t)k * n + c] = kb * ge[k] + gsc * gd[k];
+}
+__device__ inline void ee_contact(int t, const int* __restrict__ dc, int n, const int4* __restrict__ ee_set,
+                                  const int2* __restrict__ ee_ie, const int2* __restrict__ se, const double* __restrict__ x,
+                                  const double* __restrict__ vrest, double hhat, Kap kap, double* __restrict__ Hs, double* __restrict__ Gs,
+                                  int4* __restrict__ verts, int* __restrict__ dims) {
     int n_self;
     const int nc = record_contacts(dc, n_self);
-    const int c = n_self + (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int c = n_self + t;
     if (c >= nc) return;
-    double H[144];
-    {
-        const int i = c - n_self;
-        const int4 e = ee_set[i];
-        int v[4];
-        const int type = decode(e, v);
-        const double kappa = kap.at(v[0]);
-        const int nvd = nv_of(type);
-        int e4[4];
-        if (e.w >= 0) { e4[0] = e.x; e4[1] = e.y; e4[2] = e.z; e4[3] = e.w; }
-        else {
-            const int2 ie = ee_ie[i];
-            const int2 a = se[ie.x], b = se[ie.y];
-            e4[0] = a.x; e4[1] = a.y; e4[2] = b.x; e4[3] = b.y;
-        }
-        d3 p[4], pe[4];
-        for (int k = 0; k < nvd; ++k) p[k] = ld3(x, v[k]);
-        for (int k = 0; k < 4; ++k) pe[k] = ld3(x, e4[k]);
-        const double d = self_value(type, p);
-        const double b = barrier_b(d, hhat), gb = barrier_g(d, hhat), hb = barrier_h(d, hhat);
-        const double ex = eps_x_of(ld3(vrest, e4[0]), ld3(vrest, e4[1]), ld3(vrest, e4[2]), ld3(vrest, e4[3]));
-        const double cr = ee_cross_sqn(pe[0], pe[1], pe[2], pe[3]);
-        const double mol = mol_e(cr, ex);
-        // distance gradient/Hessian embedded over e4 (indMap of ContactMechanics.cpp:3627-3685)
-        double qd[12];
-        for (int k = 0; k < nvd; ++k) { qd[3 * k] = p[k].x; qd[3 * k + 1] = p[k].y; qd[3 * k + 2] = p[k].z; }
-        double gl[12];
-        dist_gh(type, qd, gl, H);
-        int map[4] = {0, 1, 2, 3};
-        if (type != 3) {
-            for (int k = 0; k < 4; ++k) {
-                if (v[0] == e4[k]) map[0] = k;
-                else if (v[1] == e4[k]) map[1] = k;
-                else if (nvd == 3 && v[2] == e4[k]) map[2] = k;
-            }
-        }
-        const int Nd = 3 * nvd;
-        double gd[12];
-        for (int k = 0; k < 12; ++k) gd[k] = 0.0;
-        for (int a = 0; a < nvd; ++a)
-            for (int r = 0; r < 3; ++r) gd[3 * map[a] + r] = gl[3 * a + r];
-        // mollifier gradient and Hessian of the cross norm
-        double qe[12], gc[12], Hc[144];
-        for (int k = 0; k < 4; ++k) { qe[3 * k] = pe[k].x; qe[3 * k + 1] = pe[k].y; qe[3 * k + 2] = pe[k].z; }
-        ee_cross_gh(qe, gc, Hc);
-        double ge[12], qg = 0.0, qH = 0.0;
-        const bool act = cr < ex;
-        if (act) {
-            const double oe = 1.0 / ex;
-            qg = 2.0 * oe * (-oe * cr + 1.0);
-            qH = -2.0 / (ex * ex);
-        }
-        for (int k = 0; k < 12; ++k) ge[k] = act ? gc[k] * qg : 0.0;
-        const double kgb = kappa * gb, kb = kappa * b, keh = kappa * mol * hb, keg = kappa * mol * gb;
-        int idx = 0;
-        for (int r = 0; r < 12; ++r)
-            for (int s = r; s < 12; ++s) {
-                // embedded distance Hessian entry
-                double hd = 0.0;
-                const int vr = r / 3, vs = s / 3;
-                int lr = -1, ls = -1;
-                for (int a = 0; a < nvd; ++a) { if (map[a] == vr) lr = a; if (map[a] == vs) ls = a; }
-                if (lr >= 0 && ls >= 0) hd = H[(3 * lr + r % 3) * Nd + 3 * ls + s % 3];
-                const double eH = act ? Hc[r * 12 + s] * qg + (qH * gc[r]) * gc[s] : 0.0;
-                const double kgg = (kgb * gd[r]) * ge[s];
-                const double kggT = (kgb * gd[s]) * ge[r];
-                Hs[(size_t)(idx++) * n + c] = kgg + kggT + kb * eH + (keh * gd[r]) * gd[s] + keg * hd;
-            }
-        const double gsc = kappa * (gb * mol);
-        for (int k = 0; k < 12; ++k) Gs[(size_t)k * n + c] = kb * ge[k] + gsc * gd[k];
-        verts[c] = make_int4(e4[0], e4[1], e4[2], e4[3]);
-        dims[c] = 12;
+    const int4 e = ee_set[t];
+    int v[4], e4[4];
+    const int type = decode(e, v);
+    const double kappa = kap.at(v[0]);
+    if (e.w >= 0) { e4[0] = e.x; e4[1] = e.y; e4[2] = e.z; e4[3] = e.w; }
+    else {
+        const int2 ie = ee_ie[t];
+        const int2 a = se[ie.x], b = se[ie.y];
+        e4[0] = a.x; e4[1] = a.y; e4[2] = b.x; e4[3] = b.y;
     }
+    switch (type) {
+    case 0: ee_local<0>(c, n, v, e4, x, vrest, hhat, kappa, Hs, Gs); break;
+    case 1: ee_local<1>(c, n, v, e4, x, vrest, hhat, kappa, Hs, Gs); break;
+    default: ee_local<3>(c, n, v, e4, x, vrest, hhat, kappa, Hs, Gs); break;
+    }
+    verts[c] = make_int4(e4[0], e4[1], e4[2], e4[3]);
+    dims[c] = 12;
+}
+// Both in one launch: row y = 0 of work-groups the Self_EE_ActiveSet contacts (the longer chain
+// first), y = 1 the Self_ActiveSet ones.
+__global__ __launch_bounds__(64) void contact_local_kernel(
+    const int* __restrict__ dc, int n, const int4* __restrict__ self_set, const int4* __restrict__ ee_set, const int2* __restrict__ ee_ie,
+    const int2* __restrict__ se, const double* __restrict__ x, const double* __restrict__ vrest, double hhat, Kap kap,
+    double* __restrict__ Hs, double* __restrict__ Gs, int4* __restrict__ verts, int* __restrict__ dims) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (blockIdx.y == 0) ee_contact(t, dc, n, ee_set, ee_ie, se, x, vrest, hhat, kap, Hs, Gs, verts, dims);
+    else self_contact(t, dc, n, self_set, x, hhat, kap, Hs, Gs, verts, dims);
 }
 
 // Kernel 2: makePD of each local Hessian, in place, one launch per vertex count and kind,
@@ -232,13 +271,23 @@ __global__ __launch_bounds__(64) void contact_pd_kernel(const int* __restrict__ 
                                                         double* __restrict__ Hs, const double* __restrict__ Gs) {
     contact_pd<M, Structured>(blockIdx.x * blockDim.x + threadIdx.x, dc, range, n, dims, Hs, Gs);
 }
-// Both 4-vertex kinds in one launch (the same registers either way): row y = 0 of work-groups
-// the Self_ActiveSet contacts (structured basis), y = 1 the Self_EE_ActiveSet ones.
+// Both 4-vertex kinds in one launch: row y = 0 of work-groups the Self_EE_ActiveSet contacts (16
+// lanes each: the longest chain first), y = 1 the Self_ActiveSet ones (structured basis).
 __global__ __launch_bounds__(64) void contact_pd4_kernel(const int* __restrict__ dc, int n, const int* __restrict__ dims,
                                                          double* __restrict__ Hs, const double* __restrict__ Gs) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (blockIdx.y == 0) contact_pd<4, true>(t, dc, 0, n, dims, Hs, Gs);
-    else contact_pd<4, false>(t, dc, 1, n, dims, Hs, Gs);
+    __shared__ double lds[4][12][9];
+    if (blockIdx.y == 1) {
+        contact_pd<4, true>(blockIdx.x * blockDim.x + threadIdx.x, dc, 0, n, dims, Hs, Gs);
+        return;
+    }
+    int ns;
+    const int nc = record_contacts(dc, ns), g = threadIdx.x >> 4;
+    for (int c0 = ns + 4 * blockIdx.x; c0 < nc; c0 += 4 * gridDim.x) {
+        const int c = c0 + g;
+        double* h = Hs + (c < nc ? c : c0);
+        project_contact_row(c < nc, [&](int k) -> double& { return h[(size_t)k * n]; }, lds[g]);
+        row_order();   // the LDS is the next block's
+    }
 }
 
 // Where the records go (sparse.hip): keys, values and bucket slots of block and gradient records.
@@ -770,10 +819,8 @@ void contact_assemble(Context& c, double kappa, bool friction_launched) {
     }
     double* Hs = c.chess.p;
     double* Gs = c.chess.p + (size_t)kHU * capS;
-    hipLaunchKernelGGL(contact_self_kernel, dim3(blocks_for(capS, 64)), dim3(64), 0, c.stream, dc, capS, c.self_set.p, s.x.p, s.hhat,
-                       scene_kappa(s, kappa), Hs, Gs, c.cverts.p, c.cdims.p);
-    hipLaunchKernelGGL(contact_ee_kernel, dim3(blocks_for(capS, 64)), dim3(64), 0, c.stream, dc, capS, c.ee_set.p, c.ee_ie.p, s.se.p,
-                       s.x.p, s.vrest.p, s.hhat, scene_kappa(s, kappa), Hs, Gs, c.cverts.p, c.cdims.p);
+    hipLaunchKernelGGL(contact_local_kernel, dim3(blocks_for(capS, 64), 2), dim3(64), 0, c.stream, dc, capS, c.self_set.p, c.ee_set.p,
+                       c.ee_ie.p, s.se.p, s.x.p, s.vrest.p, s.hhat, scene_kappa(s, kappa), Hs, Gs, c.cverts.p, c.cdims.p);
     CIPC_CHECK_LAUNCH();
     // Main stream: the projections of 4-vertex contacts.  Second stream (enqueued after them,
     // so that the main stream never waits on the host): the friction records, then the
@@ -847,20 +894,35 @@ __global__ __launch_bounds__(64) void contact_pd_eval_kernel(int n, double* __re
     double* h = H + (size_t)N * N * t;
     auto acc = [&](int k) -> double& { return h[Sym<N>::row(k) * N + Sym<N>::col(k)]; };
     bool changed;
+    auto general = [&] {
+        if constexpr (M == 4) return false;   // contact_pd_row_eval_kernel
+        else return project_contact<M>(acc);
+    };
     if constexpr (M >= 3) {
         if (G != nullptr) {
             double g[N];
             for (int k = 0; k < N; ++k) g[k] = G[(size_t)N * t + k];
             changed = project_contact_structured<M>(acc, g);
         } else {
-            changed = project_contact<M>(acc);
+            changed = general();
         }
     } else {
-        changed = project_contact<M>(acc);
+        changed = general();
     }
     if (!changed) return;
     for (int i = 0; i < N; ++i)
         for (int j = i + 1; j < N; ++j) h[j * N + i] = h[i * N + j];
+}
+// The general 4-vertex projection as the assembly runs it: 16 lanes per block.
+__global__ __launch_bounds__(64) void contact_pd_row_eval_kernel(int n, double* __restrict__ H) {
+    __shared__ double lds[4][12][9];
+    const int g = threadIdx.x >> 4, t = 4 * blockIdx.x + g;
+    double* h = H + 144 * (size_t)(t < n ? t : 0);
+    project_contact_row(t < n, [&](int k) -> double& { return h[Sym<12>::row(k) * 12 + Sym<12>::col(k)]; }, lds[g]);
+    __syncthreads();
+    if (t < n && (threadIdx.x & 15) == 0)
+        for (int i = 0; i < 12; ++i)
+            for (int j = i + 1; j < 12; ++j) h[j * 12 + i] = h[i * 12 + j];
 }
 __global__ void accd_eval_kernel(int n, int kind, const double* __restrict__ pts, const double* __restrict__ dirs, double eta,
                                  double th, double* __restrict__ toc) {
@@ -918,7 +980,8 @@ extern "C" int cipc_gpu_eval_contact_pd_impl(int n, int nverts, double* H, const
     const double* gp = G ? dg.p : nullptr;
     if (nverts == 2) hipLaunchKernelGGL(contact_pd_eval_kernel<2>, dim3(blocks_for(n, 64)), dim3(64), 0, 0, n, dh.p, gp);
     else if (nverts == 3) hipLaunchKernelGGL(contact_pd_eval_kernel<3>, dim3(blocks_for(n, 64)), dim3(64), 0, 0, n, dh.p, gp);
-    else hipLaunchKernelGGL(contact_pd_eval_kernel<4>, dim3(blocks_for(n, 64)), dim3(64), 0, 0, n, dh.p, gp);
+    else if (gp) hipLaunchKernelGGL(contact_pd_eval_kernel<4>, dim3(blocks_for(n, 64)), dim3(64), 0, 0, n, dh.p, gp);
+    else hipLaunchKernelGGL(contact_pd_row_eval_kernel, dim3(blocks_for(n, 4)), dim3(64), 0, 0, n, dh.p);
     CIPC_CHECK_LAUNCH();
     dh.down(H, dim * dim * n);
     return 0;

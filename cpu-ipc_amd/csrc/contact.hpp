@@ -271,6 +271,30 @@ __device__ constexpr double helmert(int M, int i, int a) {
 // Circle-method round robin over NP (even) indices: pair i of round r.
 __device__ constexpr int rr_slot(int NP, int r, int k) { return k == 0 ? 0 : ((k - 1 + r) % (NP - 1)) + 1; }
 
+// 1 / x and 1 / sqrt(x) to about an ulp for normal x: the hardware's estimate and two Newton steps,
+// a third of the instructions of the correctly rounded division and root.
+__device__ inline double fast_rcp(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+    return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+__device__ inline double fast_rsqrt(double x) {
+    double r = __builtin_amdgcn_rsq(x);
+    r = __builtin_fma(__builtin_fma(-x * r, r, 1.0), 0.5 * r, r);
+    return __builtin_fma(__builtin_fma(-x * r, r, 1.0), 0.5 * r, r);
+}
+// The Jacobi rotation of (app, apq, aqq): t, c, s = t c; t = 0 for an entry of no weight.  An
+// inexact t only leaves a remainder of the order of the rounding (c is made from it); the
+// bound on |theta| keeps its square finite.
+__device__ inline void jacobi_angle(double app, double apq, double aqq, double& t, double& c, double& s) {
+    const bool zero = !(fabs(apq) > 1e-290);
+    const double th = 0.5 * (aqq - app) * fast_rcp(zero ? 1.0 : apq);
+    const double m = fmin(fabs(th), 1e100), x = __builtin_fma(m, m, 1.0);
+    t = fast_rcp(__builtin_fma(x, fast_rsqrt(x), m));
+    t = zero ? 0.0 : th < 0.0 ? -t : t;
+    c = fast_rsqrt(__builtin_fma(t, t, 1.0));
+    s = t * c;
+}
 // Cyclic-by-rounds Jacobi on the packed upper triangle R (Sym<NR>) with eigenvectors Z
 // (row-major NR x NR, columns are eigenvectors).  Each round rotates NP/2 disjoint pairs whose
 // angles depend only on entries no other pair of the round touches, so the angles of a round
@@ -301,15 +325,11 @@ __device__ inline void jacobi_rounds(double* __restrict__ R, double* __restrict_
                 if (q >= NR) continue;
                 const double apq = R[Sym<NR>::ix(p, q)];
                 const double app = R[Sym<NR>::ix(p, p)], aqq = R[Sym<NR>::ix(q, q)];
-                const bool zero = apq == 0.0;
-                const double th = (aqq - app) / (zero ? 1.0 : 2.0 * apq);
-                double t = (th >= 0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
-                t = zero ? 0.0 : t;
-                const double c = 1.0 / sqrt(t * t + 1.0);
-                cs[h] = c; sn[h] = t * c;
+                double t;
+                jacobi_angle(app, apq, aqq, t, cs[h], sn[h]);
                 R[Sym<NR>::ix(p, p)] = app - t * apq;
                 R[Sym<NR>::ix(q, q)] = aqq + t * apq;
-                R[Sym<NR>::ix(p, q)] = zero ? apq : 0.0;
+                R[Sym<NR>::ix(p, q)] = t == 0.0 ? apq : 0.0;
             }
 #pragma unroll
             for (int h = 0; h < NH; ++h) {
@@ -408,6 +428,179 @@ __device__ inline bool project_contact(HA h) {
         }
     lift_subtract<M>(h, R);
     return true;
+}
+
+// The general projection of a 12 x 12 block by 16 lanes (four blocks a wavefront): lane j holds
+// column j of the block and row j of its eigenvectors.  In the Jacobi rounds the two lanes of a
+// pair exchange their columns and every lane turns its rows, so a round costs one angle instead
+// of four and an eighth of the updates.  One lane per block took 100 us whatever their number,
+// and the mollified edge-edge blocks are few, so that was the length of the stage: 150 -> 44 us on four 20^3 cubes (876 of 14,085 contacts),
+// 199 -> 107 on four 32^3.
+// h(k): packed entry of the lane's block; active: the same in the 16 lanes; lds: 12 x 9 doubles of
+// the block.  All 64 lanes call it.
+__device__ inline double row_lane(double v, int lane16) {   // lane16's value in each row of 16 lanes, lane16 lane-dependent
+    const int src = ((threadIdx.x & 48) | lane16) << 2;
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_ds_bpermute(src, (int)b), hi = __builtin_amdgcn_ds_bpermute(src, (int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | lo);
+}
+template <int L>
+__device__ inline double row_bcast(double v) {              // lane L's value in each row of 16 lanes
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x150 + L, 0xf, 0xf, true);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x150 + L, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | lo);
+}
+template <int D>
+__device__ inline double row_rotate(double v) {             // the value D lanes on in the row of 16
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x120 + D, 0xf, 0xf, true);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x120 + D, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | lo);
+}
+__device__ inline double row_total(double v) {              // the sum over the row of 16 lanes, in each of them
+    v += row_rotate<8>(v);
+    v += row_rotate<4>(v);
+    v += row_rotate<2>(v);
+    return v + row_rotate<1>(v);
+}
+__device__ inline void row_order() {                        // order of a wavefront's own LDS accesses
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+template <int Q, int H>
+__device__ inline void row_pair(int lane, double (&r)[9], double (&z)[9], double c, double s, double t) {
+    constexpr int a = rr_slot(10, Q, H), b = rr_slot(10, Q, 9 - H), p = a < b ? a : b, q = a < b ? b : a;
+    if constexpr (q < 9) {
+        const double cp = row_bcast<p>(c), sp = row_bcast<p>(s);
+        const double rp = r[p], rq = r[q], zp = z[p], zq = z[q];
+        r[p] = cp * rp - sp * rq;
+        r[q] = sp * rp + cp * rq;
+        z[p] = cp * zp - sp * zq;
+        z[q] = sp * zp + cp * zq;
+        // the pair's own entry is annihilated (its diagonal entries are kept apart)
+        if (lane == p && t != 0.0) r[q] = 0.0;
+        if (lane == q && t != 0.0) r[p] = 0.0;
+    }
+}
+template <int Q>
+__device__ inline void row_round(int lane, double (&r)[9], double (&z)[9], double& dg) {
+    // the lane's partner in round Q and the entry it shares with it
+    int m = lane;
+    double apq = 0.0;
+#pragma unroll
+    for (int h = 0; h < 5; ++h) {
+        const int a = rr_slot(10, Q, h), b = rr_slot(10, Q, 9 - h), p = a < b ? a : b, q = a < b ? b : a;
+        if (q >= 9) continue;
+        if (lane == p) { m = q; apq = r[q]; }
+        if (lane == q) { m = p; apq = r[p]; }
+    }
+    const double dm = row_lane(dg, m);
+    const bool first = lane < m;
+    // the first lane's copy of the shared entry: the two round apart, and where the diagonal
+    // entries are close the angle is all in its sign and size
+    apq = row_lane(apq, first ? lane : m);
+    double t, c, s;
+    jacobi_angle(first ? dg : dm, apq, first ? dm : dg, t, c, s);
+    dg += first ? -t * apq : t * apq;
+    const double so = first ? -s : s;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) r[k] = c * r[k] + so * row_lane(r[k], m);
+    row_pair<Q, 0>(lane, r, z, c, s, t);
+    row_pair<Q, 1>(lane, r, z, c, s, t);
+    row_pair<Q, 2>(lane, r, z, c, s, t);
+    row_pair<Q, 3>(lane, r, z, c, s, t);
+    row_pair<Q, 4>(lane, r, z, c, s, t);
+}
+template <typename HA>
+__device__ inline void project_contact_row(bool active, HA h, double (*__restrict__ lds)[9]) {
+    const int lane = threadIdx.x & 15, l = lane % 3;
+    double col[12], r[9], z[9];
+#pragma unroll
+    for (int k = 0; k < 12; ++k) col[k] = active && lane < 12 ? h(Sym<12>::ix(k, lane)) : 0.0;
+    // R = B H B^T: rows in the lane, columns through LDS
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            double acc = 0.0;
+#pragma unroll
+            for (int a = 0; a <= i + 1; ++a) acc += helmert(4, i, a) * col[3 * a + k];
+            if (lane < 12) lds[lane][3 * i + k] = acc;
+        }
+    row_order();
+    const int j = lane / 3;
+    double hm[4];   // Helmert row j
+#pragma unroll
+    for (int a = 0; a < 4; ++a) hm[a] = j == 0 ? helmert(4, 0, a) : j == 1 ? helmert(4, 1, a) : helmert(4, 2, a);
+    double dg = 0.0;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        double acc = 0.0;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc += hm[b] * lds[3 * b + l][k];
+        r[k] = lane < 9 ? acc : 0.0;
+        z[k] = lane == k ? 1.0 : 0.0;
+        dg = lane == k ? r[k] : dg;
+    }
+    for (int sweep = 0; sweep < 32; ++sweep) {
+        double off = 0.0;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) off += lane == k ? 0.0 : r[k] * r[k];
+        off = row_total(off);
+        const double d2 = row_total(dg * dg);
+        if (!__any(active && !(off == 0.0 || off <= 2e-30 * d2))) break;   // (off counts every entry twice)
+        row_round<0>(lane, r, z, dg); row_round<1>(lane, r, z, dg); row_round<2>(lane, r, z, dg);
+        row_round<3>(lane, r, z, dg); row_round<4>(lane, r, z, dg); row_round<5>(lane, r, z, dg);
+        row_round<6>(lane, r, z, dg); row_round<7>(lane, r, z, dg); row_round<8>(lane, r, z, dg);
+    }
+    const double w = lane < 9 ? fmin(dg, 0.0) : 0.0;
+    const unsigned long long neg = __ballot(active && w < 0.0);
+    const bool mine = (neg >> (threadIdx.x & 48)) & 0xffffull;   // a block without negative eigenvalues stays as it is
+    if (!neg) return;
+    // column `lane` of the negative part: N(k, lane) = sum_j w_j Z(lane, j) Z(k, j)
+    row_order();
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+        if (lane < 9) lds[lane][k] = z[k];
+    row_order();
+    double n[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 9; ++j) {
+        if (!(neg & (0x0001000100010001ull << j))) continue;
+        const double x = row_lane(w, j) * z[j];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) n[k] += x * lds[k][j];
+    }
+    row_order();
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+        if (lane < 9) lds[lane][k] = n[k];
+    row_order();
+    // H -= B^T N B: column (b, l) of N B, then its rows
+    const int b = lane / 3;
+    double x[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        double acc = 0.0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const double e = b == 0 ? helmert(4, i, 0) : b == 1 ? helmert(4, i, 1) : b == 2 ? helmert(4, i, 2) : helmert(4, i, 3);
+            acc += e * lds[3 * i + l][k];
+        }
+        x[k] = acc;
+    }
+    if (!mine || lane >= 12) return;
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            double acc = 0.0;
+#pragma unroll
+            for (int i = (a > 0 ? a - 1 : 0); i < 3; ++i) acc += helmert(4, i, a) * x[3 * i + k];
+            if (3 * a + k <= lane) h(Sym<12>::ix(3 * a + k, lane)) = col[3 * a + k] - acc;
+        }
 }
 
 // ---- Structured contact blocks: a smaller eigenproblem on the block's range.

@@ -195,6 +195,7 @@ struct Context {
     DBuf<int> fdims;
     DBuf<int4> fverts;
 
+    DBuf<double> hingeH;       // hinge blocks before their projection (packed upper triangle, SoA)
     // contact contributions (fixed slots, invalid key = ~0ull)
     DBuf<unsigned long long> ckey;
     DBuf<double> cval;         // 9 per record
