@@ -4,6 +4,7 @@
 #include "common.hpp"
 
 #include <cstring>
+#include <initializer_list>
 #include <limits>
 
 namespace cipc {
@@ -111,6 +112,8 @@ struct SolveResult {
 };
 
 struct LearnedState;
+
+constexpr int kReadSlots = 4;   // staging of read_arrays
 
 struct Context {
     int device = 0;
@@ -229,6 +232,10 @@ struct Context {
     PinnedBuf<int> pin_nnz;
     PinnedBuf<int> pin_as;     // counts of the active-set construction
     PinnedBuf<unsigned char> pin_rb;   // staging of read_back
+    // staging of read_arrays: kReadSlots slots of read_chunk bytes, an event for each
+    PinnedBuf<unsigned char> pin_arrays;
+    size_t read_chunk = 0;
+    hipEvent_t read_ev[kReadSlots] = {};
     PinnedBuf<unsigned long long> pin_slots;
     PinnedBuf<double> pin_energy;
     PinnedBuf<int> pin_pcg;            // a solve's progress, written by its kernels
@@ -263,6 +270,16 @@ void read_back(Context& c, T* host, const T* dev, size_t n) {
     CIPC_HIP(hipStreamSynchronize(c.stream));
     std::memcpy(static_cast<void*>(host), c.pin_rb.p, n * sizeof(T));
 }
+
+// Arrays from the device to the caller's pageable memory, after the stream's pending work;
+// returns once they are there.  Null or empty ones are skipped.
+struct HostArray {
+    void* host;
+    const void* dev;
+    size_t bytes;
+};
+void read_arrays_prepare(Context& c, size_t largest);
+void read_arrays(Context& c, std::initializer_list<HostArray> arrays);
 
 // elastic.hip
 void build_static_pattern(Context& c);
