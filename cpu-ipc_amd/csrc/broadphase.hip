@@ -662,68 +662,85 @@ __device__ inline void ee_classify(int u, const int* __restrict__ dc, int Es, co
     }
 }
 
-// Per-category output positions: one exclusive scan of four 0/1 category counts per hit
-// (int4 x, y, z, w).
-struct Cnt4Sum {
-    __host__ __device__ int4 operator()(const int4& p, const int4& q) const { return make_int4(p.x + q.x, p.y + q.y, p.z + q.z, p.w + q.w); }
-};
-// Both hit kinds in one scan: items [0, n1) the point-triangle hits (dc[kDcPT] of them), the
-// rest the edge-edge hits (dc[kDcEE]), each with its own category masks; nothing is counted
-// over capacity.
-struct CatFlags {
-    const int* catPT;
-    const int* catEE;
-    const int* dc;
-    int n1;
-    unsigned a0, a1, a2, a3, b0, b1, b2, b3;
-    __host__ __device__ int4 operator()(int i) const {
-        if (dc[kDcFlags]) return make_int4(0, 0, 0, 0);
-        const bool pt = i < n1;
-        const int j = pt ? i : i - n1;
-        if (j >= dc[pt ? kDcPT : kDcEE]) return make_int4(0, 0, 0, 0);
-        const unsigned bit = 1u << (pt ? catPT : catEE)[j];
-        const unsigned m0 = pt ? a0 : b0, m1 = pt ? a1 : b1, m2 = pt ? a2 : b2, m3 = pt ? a3 : b3;
-        return make_int4((m0 & bit) ? 1 : 0, (m1 & bit) ? 1 : 0, (m2 & bit) ? 1 : 0, (m3 & bit) ? 1 : 0);
+// Per-category output positions of the hits (four 0/1 categories each, int4 x, y, z, w): the
+// counts of every kCatBlock hits, which the scatter's work-groups then add up themselves, each to
+// its own block, and ballots within a block.  Only the hits there are, not the capacity, are
+// read, and no position is stored: a device-wide scan over the capacities wrote 16 bytes a
+// slot (with the scatter 333 us on a batch of 40 scenes and 55 on a folded 128^2 cloth, now 110 and 19).
+constexpr int kCatBlock = 1024, kCatThreads = 256;
+// Category masks of the point-triangle hits and of the edge-edge hits.
+__device__ constexpr unsigned kCatPT[4] = {1u << kSelfPT, 1u << kMap, (1u << kNone) | (1u << kSelfPT) | (1u << kMap), 0u};
+__device__ constexpr unsigned kCatEE[4] = {1u << kSelfEE, 1u << kMap, (1u << kMolPE) | (1u << kMolEE),
+                                           (1u << kNone) | (1u << kSelfEE) | (1u << kMap) | (1u << kMolPE) | (1u << kMolEE)};
+template <bool Pt>
+__device__ inline int cat_count(int c, unsigned bit, unsigned long long& m) {
+    m = __ballot((Pt ? kCatPT[c] : kCatEE[c]) & bit);
+    return __popcll(m);
+}
+// The counts of a wavefront's hits [i0, i0 + kCatBlock / 4).
+template <bool Pt>
+__device__ inline int4 wave_counts(const int* __restrict__ cat, int i0, int n) {
+    int4 t = make_int4(0, 0, 0, 0);
+    unsigned long long m;
+#pragma unroll
+    for (int r = 0; r < kCatBlock / kCatThreads; ++r) {
+        const int i = i0 + 64 * r + (threadIdx.x & 63);
+        const unsigned bit = i < n ? 1u << cat[i] : 0u;
+        t.x += cat_count<Pt>(0, bit, m);
+        t.y += cat_count<Pt>(1, bit, m);
+        t.z += cat_count<Pt>(2, bit, m);
+        t.w += cat_count<Pt>(3, bit, m);
     }
-};
+    return t;
+}
+__device__ inline int4 add4(int4 p, int4 q) { return make_int4(p.x + q.x, p.y + q.y, p.z + q.z, p.w + q.w); }
+__device__ inline int4 wave_add4(int4 v) {
+    for (int d = 32; d > 0; d >>= 1)
+        v = add4(v, make_int4(__shfl_xor(v.x, d), __shfl_xor(v.y, d), __shfl_xor(v.z, d), __shfl_xor(v.w, d)));
+    return v;
+}
+// Work-groups [0, bPT) the point hits' blocks, the rest the edge hits' (sums from bPT on).
+__global__ __launch_bounds__(kCatThreads) void category_counts(const int* __restrict__ dc, int bPT, const int* __restrict__ catPT,
+                                                               const int* __restrict__ catEE, int4* __restrict__ sums) {
+    __shared__ int4 sh[kCatThreads / 64];
+    if (dc[kDcFlags]) return;
+    const bool pt = (int)blockIdx.x < bPT;
+    const int b = pt ? blockIdx.x : blockIdx.x - bPT, n = dc[pt ? kDcPT : kDcEE], w = threadIdx.x >> 6;
+    if (b * kCatBlock >= n) return;
+    const int i0 = b * kCatBlock + w * (kCatBlock / 4);
+    const int4 t = pt ? wave_counts<true>(catPT, i0, n) : wave_counts<false>(catEE, i0, n);
+    if ((threadIdx.x & 63) == 0) sh[w] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) sums[blockIdx.x] = add4(add4(sh[0], sh[1]), add4(sh[2], sh[3]));
+}
 // PP/PE map key: (c0 + V, c1, c2 + 1) packed with `bits` per field preserves the signed
 // lexicographic order of std::map<EncodedContact, int> (all keys have c3 = -1).
 __device__ inline unsigned long long map_key(int4 r, int V, int bits) {
     return ((unsigned long long)(r.x + V) << (2 * bits)) | ((unsigned long long)r.y << bits) | (unsigned long long)(r.z + 1);
 }
-// Point-triangle hits -> Self_ActiveSet head (a), map keys (b), partial-CCD pairs (c).
-__device__ inline void scatter_pt(int i, int nPT, const int* __restrict__ cat, const int4* __restrict__ pos,
-                                  const int4* __restrict__ rec, const int* __restrict__ own, const int* __restrict__ cand, int V, int bits,
-                                  int4* __restrict__ self_set, unsigned long long* __restrict__ mkeys, int2* __restrict__ ccd) {
-    if (i >= nPT) return;
-    const int ct = cat[i];
+// Point-triangle hit i at positions p -> Self_ActiveSet head (a), map keys (b), partial-CCD pairs (c).
+__device__ inline void scatter_pt(int i, int ct, int4 p, const int4* __restrict__ rec, const int* __restrict__ own,
+                                  const int* __restrict__ cand, int V, int bits, int4* __restrict__ self_set,
+                                  unsigned long long* __restrict__ mkeys, int2* __restrict__ ccd) {
     if (ct == kDrop) return;
-    const int4 p = pos[i];
     ccd[p.z] = make_int2(-own[i] - 1, cand[i]);
     if (ct == kSelfPT) self_set[p.x] = rec[i];
     else if (ct == kMap) mkeys[p.y] = map_key(rec[i], V, bits);
 }
-// Edge-edge hits -> Self_ActiveSet (a), map keys (b), Self_EE_ActiveSet + eIe (c), CCD pairs (d).
+// Edge-edge hit i -> Self_ActiveSet (a), map keys (b), Self_EE_ActiveSet + eIe (c), CCD pairs (d).
 // base: the point hits' totals (Self_ActiveSet, map keys, CCD pairs), where the edge hits'
 // entries start.
-__device__ inline void scatter_ee(int i, int nEE, int4 base, const int* __restrict__ cat, const int4* __restrict__ pos,
-                                  const int4* __restrict__ rec, const int2* __restrict__ aux, const int* __restrict__ own,
-                                  const int* __restrict__ cand, int V, int bits, int4* __restrict__ self_set,
-                                  unsigned long long* __restrict__ mkeys, int4* __restrict__ ee_set, int2* __restrict__ ee_ie,
-                                  int2* __restrict__ ccd) {
-    if (i >= nEE) return;
-    const int base_self = base.x, base_map = base.y, base_ccd = base.z;
-    const int ct = cat[i];
+__device__ inline void scatter_ee(int i, int ct, int4 p, int4 base, const int4* __restrict__ rec, const int2* __restrict__ aux,
+                                  const int* __restrict__ own, const int* __restrict__ cand, int V, int bits,
+                                  int4* __restrict__ self_set, unsigned long long* __restrict__ mkeys, int4* __restrict__ ee_set,
+                                  int2* __restrict__ ee_ie, int2* __restrict__ ccd) {
     if (ct == kDrop) return;
-    const int4 q = pos[i], z = pos[0];   // the joint scan's edge segment starts at the point totals
-    const int4 p = make_int4(q.x - z.x, q.y - z.y, q.z - z.z, q.w - z.w);
-    ccd[base_ccd + p.w] = make_int2(own[i], cand[i]);
-    if (ct == kSelfEE) self_set[base_self + p.x] = rec[i];
-    else if (ct == kMap) mkeys[base_map + p.y] = map_key(rec[i], V, bits);
+    ccd[base.z + p.w] = make_int2(own[i], cand[i]);
+    if (ct == kSelfEE) self_set[base.x + p.x] = rec[i];
+    else if (ct == kMap) mkeys[base.y + p.y] = map_key(rec[i], V, bits);
     else if (ct == kMolPE || ct == kMolEE) { ee_set[p.z] = rec[i]; ee_ie[p.z] = aux[i]; }
 }
-// Counts after the category scans: the per-category totals are the scans' values at the hit
-// counts, the ground count the ground scan's total.  The map keys fill [0, nm) of a
+// Counts: the per-category totals of both kinds, the ground count the ground scan's total.  The map keys fill [0, nm) of a
 // buffer of capM; past nm they are the all-ones key, which sorts last.
 __device__ inline void category_totals(int Vs, const int4& a, const int4& b, const int* __restrict__ pg, int capM, int* __restrict__ dc) {
     const int nm = a.y + b.y;
@@ -760,61 +777,92 @@ __device__ inline void ground_scatter(int s, int Vs, const int* __restrict__ sv,
     if (s >= Vs || !flag[s]) return;
     out[pos[s] - pos[0]] = sv[s];
 }
-// After the category scan, in one launch (the four parts write disjoint entries): work-groups
-// [0, bPT) place the point hits, the next bEE the edge hits, the next bG the ground entries,
-// the rest write the map keys' all-ones tail.  Every thread reads the per-category totals
-// (the scan's values at the hit counts) itself; the first publishes them (category_totals).
-// Nothing is placed when a capacity was exceeded: the host builds the set again.
+// In one launch (the four parts write disjoint entries): work-groups [0, bPT) place the point
+// hits, the next bEE the edge hits, the next bG the ground entries, the rest write the map keys'
+// all-ones tail.  Every work-group with work adds up the blocks' counts; the first publishes the
+// totals (category_totals).  Nothing is placed when a capacity was exceeded: the host builds the
+// set again.
 struct ScatterArgs {
     int* dc;
     int V, bits, Vs, capM, bPT, bEE, bG;
     const int *catPT, *ownPT, *candPT, *catEE, *ownEE, *candEE, *sv, *fg, *pg;
-    const int4 *posPT, *recPT, *posEE, *recEE;
+    const int4 *sums, *recPT, *recEE;
     const int2* auxEE;
     int4 *self_set, *ee_set;
     int2 *ee_ie, *ccd;
     unsigned long long* mkeys;
     int* env;
 };
-__global__ void scatter_all(ScatterArgs a) {
+// A block's hits with their positions: put(hit, category, position).
+template <bool Pt, typename P>
+__device__ inline void place_hits(const int* __restrict__ cat, int b, int n, int4 at, int4* sh, P&& put) {
+    const int w = threadIdx.x >> 6, i0 = b * kCatBlock + w * (kCatBlock / 4);
+    const int4 t = wave_counts<Pt>(cat, i0, n);
+    if ((threadIdx.x & 63) == 0) sh[w] = t;
+    __syncthreads();
+    for (int k = 0; k < w; ++k) at = add4(at, sh[k]);
+    const unsigned long long before = (1ull << (threadIdx.x & 63)) - 1;
+#pragma unroll
+    for (int r = 0; r < kCatBlock / kCatThreads; ++r) {
+        const int i = i0 + 64 * r + (threadIdx.x & 63);
+        const int ct = i < n ? cat[i] : kDrop;
+        const unsigned bit = i < n ? 1u << ct : 0u;
+        unsigned long long m0, m1, m2, m3;
+        const int4 c = make_int4(cat_count<Pt>(0, bit, m0), cat_count<Pt>(1, bit, m1), cat_count<Pt>(2, bit, m2), cat_count<Pt>(3, bit, m3));
+        put(i, ct, make_int4(at.x + __popcll(m0 & before), at.y + __popcll(m1 & before), at.z + __popcll(m2 & before), at.w + __popcll(m3 & before)));
+        at = add4(at, c);
+    }
+}
+__global__ __launch_bounds__(kCatThreads) void scatter_all(ScatterArgs a) {
+    __shared__ int4 sh[3][kCatThreads / 64], hits[kCatThreads / 64];
     int* dc = a.dc;
-    if (dc[kDcFlags]) return;   // the candidates exceeded their capacity (an earlier launch)
+    if (dc[kDcFlags] & 3) return;   // the candidates exceeded their capacity (an earlier launch)
     const int nPT = dc[kDcPT], nEE = dc[kDcEE];
-    const int4 ta = a.posPT[nPT], q = a.posEE[nEE], z = a.posEE[0];
-    const int4 tb = make_int4(q.x - z.x, q.y - z.y, q.z - z.z, q.w - z.w);
-    if (blockIdx.x == 0 && threadIdx.x == 0) category_totals(a.Vs, ta, tb, a.pg, a.capM, dc);
+    const int b = blockIdx.x;
+    const bool first = b == 0, pt = b < a.bPT, ee = !pt && b < a.bPT + a.bEE;
+    if (!first && ((pt && b * kCatBlock >= nPT) || (ee && (b - a.bPT) * kCatBlock >= nEE))) return;
+    // the totals of both kinds (ta, tb), and the counts before this block (of its kind)
+    int4 ta = make_int4(0, 0, 0, 0), tb = ta, at = ta;
+    {
+        const int4 zero = ta;
+        const int kPT = (nPT + kCatBlock - 1) / kCatBlock, kEE = (nEE + kCatBlock - 1) / kCatBlock;
+        for (int k = threadIdx.x; k < kPT + kEE; k += kCatThreads) {
+            const bool p = k < kPT;
+            const int block = p ? k : a.bPT + k - kPT;
+            const int4 v = a.sums[block];
+            if (p) ta = add4(ta, v);
+            else tb = add4(tb, v);
+            if (p == pt && block < b) at = add4(at, v);
+        }
+        if (!pt && !ee) at = zero;
+        ta = wave_add4(ta); tb = wave_add4(tb); at = wave_add4(at);
+        if ((threadIdx.x & 63) == 0) {
+            const int w = threadIdx.x >> 6;
+            sh[0][w] = ta; sh[1][w] = tb; sh[2][w] = at;
+        }
+        __syncthreads();
+        ta = add4(add4(sh[0][0], sh[0][1]), add4(sh[0][2], sh[0][3]));
+        tb = add4(add4(sh[1][0], sh[1][1]), add4(sh[1][2], sh[1][3]));
+        at = add4(add4(sh[2][0], sh[2][1]), add4(sh[2][2], sh[2][3]));
+    }
+    if (first && threadIdx.x == 0) category_totals(a.Vs, ta, tb, a.pg, a.capM, dc);
     const int nm = ta.y + tb.y;
     if (nm > a.capM) return;
-    int b = blockIdx.x;
-    if (b < a.bPT) {
-        scatter_pt(b * blockDim.x + threadIdx.x, nPT, a.catPT, a.posPT, a.recPT, a.ownPT, a.candPT, a.V, a.bits, a.self_set, a.mkeys,
-                   a.ccd);
+    if (pt) {
+        place_hits<true>(a.catPT, b, nPT, at, hits, [&](int i, int ct, int4 p) {
+            scatter_pt(i, ct, p, a.recPT, a.ownPT, a.candPT, a.V, a.bits, a.self_set, a.mkeys, a.ccd);
+        });
         return;
     }
-    b -= a.bPT;
-    if (b < a.bEE) {
-        scatter_ee(b * blockDim.x + threadIdx.x, nEE, ta, a.catEE, a.posEE, a.recEE, a.auxEE, a.ownEE, a.candEE, a.V, a.bits,
-                   a.self_set, a.mkeys, a.ee_set, a.ee_ie, a.ccd);
+    if (ee) {
+        place_hits<false>(a.catEE, b - a.bPT, nEE, at, hits, [&](int i, int ct, int4 p) {
+            scatter_ee(i, ct, p, ta, a.recEE, a.auxEE, a.ownEE, a.candEE, a.V, a.bits, a.self_set, a.mkeys, a.ee_set, a.ee_ie, a.ccd);
+        });
         return;
     }
-    b -= a.bEE;
-    if (b < a.bG) {
-        ground_scatter(b * blockDim.x + threadIdx.x, a.Vs, a.sv, a.fg, a.pg, a.env);
-        return;
-    }
-    b -= a.bG;
-    map_tail(b * blockDim.x + threadIdx.x, a.capM, nm, a.mkeys);
-}
-// Exclusive scan of the four category flags over n items (flags past a kind's count are
-// zero, so each kind's totals follow its last hit).
-void category_scan(Context& c, const CatFlags& f, int n, DBuf<int4>& pos) {
-    pos.resize((size_t)n + 1);
-    hipcub::CountingInputIterator<int> idx(0);
-    hipcub::TransformInputIterator<int4, CatFlags, hipcub::CountingInputIterator<int>> it(idx, f);
-    size_t bytes = 0;
-    CIPC_HIP(hipcub::DeviceScan::ExclusiveScan(nullptr, bytes, it, pos.p, Cnt4Sum(), make_int4(0, 0, 0, 0), n + 1, c.stream));
-    c.tmp.reserve(bytes);
-    CIPC_HIP(hipcub::DeviceScan::ExclusiveScan(c.tmp.p, bytes, it, pos.p, Cnt4Sum(), make_int4(0, 0, 0, 0), n + 1, c.stream));
+    const int g = b - a.bPT - a.bEE;
+    if (g < a.bG) ground_scatter(g * kCatThreads + threadIdx.x, a.Vs, a.sv, a.fg, a.pg, a.env);
+    else map_tail((g - a.bG) * kCatThreads + threadIdx.x, a.capM, nm, a.mkeys);
 }
 
 // The walks' hit buffers.
@@ -1050,18 +1098,12 @@ void compute_active_set(Context& c, bool publish) {
     launch_active_walks(c, true, true, true, c.tune.as_pt_bits, c.tune.as_ee_bits, c.stream);
     if (cl.nbp + nbe > 0) hipLaunchKernelGGL(classify_both, dim3(cl.nbp + nbe), dim3(128), 0, c.stream, cl);
     CIPC_CHECK_LAUNCH();
-    // category positions
-    const unsigned keptPT = (1u << kNone) | (1u << kSelfPT) | (1u << kMap);
-    const unsigned keptEE = (1u << kNone) | (1u << kSelfEE) | (1u << kMap) | (1u << kMolPE) | (1u << kMolEE);
-    // both kinds of hit in one scan: points [0, capPT], edges after them
-    b.pos_all.resize((size_t)capPT + 1 + capEE + 1);
-    {
-        const CatFlags f{b.catPT.p, b.catEE.p, dc, capPT + 1, 1u << kSelfPT, 1u << kMap, keptPT, 0u,
-                         1u << kSelfEE, 1u << kMap, (1u << kMolPE) | (1u << kMolEE), keptEE};
-        category_scan(c, f, capPT + 1 + capEE + 1, b.pos_all);
-    }
-    const int4* posPT = b.pos_all.p;
-    const int4* posEE = posPT + (capPT + 1);
+    // category counts of every block of hits
+    const int blocksPT = (int)blocks_for(capPT, kCatBlock), blocksEE = (int)blocks_for(capEE, kCatBlock);
+    b.cat_sums.resize((size_t)blocksPT + blocksEE);
+    hipLaunchKernelGGL(category_counts, dim3(blocksPT + blocksEE), dim3(kCatThreads), 0, c.stream, dc, blocksPT, b.catPT.p, b.catEE.p,
+                       b.cat_sums.p);
+    CIPC_CHECK_LAUNCH();
     // PP/PE map keys need the vertex count to fit three fields in 64 bits
     int bits = 1;
     while ((1ll << bits) < (long long)s.V + 2) ++bits;
@@ -1073,13 +1115,13 @@ void compute_active_set(Context& c, bool publish) {
     {
         ScatterArgs a;
         a.dc = dc; a.V = s.V; a.bits = bits; a.Vs = Vs; a.capM = capM;
-        a.bPT = (int)blocks_for(capPT, 256); a.bEE = (int)blocks_for(capEE, 256); a.bG = (int)blocks_for(Vs, 256);
-        a.catPT = b.catPT.p; a.ownPT = b.ownPT.p; a.candPT = b.candPT.p; a.posPT = posPT; a.recPT = b.recPT.p;
-        a.catEE = b.catEE.p; a.ownEE = b.ownEE.p; a.candEE = b.candEE.p; a.posEE = posEE; a.recEE = b.recEE.p; a.auxEE = b.auxEE.p;
+        a.bPT = blocksPT; a.bEE = blocksEE; a.bG = (int)blocks_for(Vs, kCatThreads); a.sums = b.cat_sums.p;
+        a.catPT = b.catPT.p; a.ownPT = b.ownPT.p; a.candPT = b.candPT.p; a.recPT = b.recPT.p;
+        a.catEE = b.catEE.p; a.ownEE = b.ownEE.p; a.candEE = b.candEE.p; a.recEE = b.recEE.p; a.auxEE = b.auxEE.p;
         a.sv = s.sv.p; a.fg = cG; a.pg = oG; a.self_set = c.self_set.p; a.ee_set = c.ee_set.p; a.ee_ie = c.ee_ie.p;
         a.ccd = c.ccd_set.p; a.mkeys = b.mkeys.p; a.env = c.env_set.p;
-        const int blocks = a.bPT + a.bEE + a.bG + (int)blocks_for(capM, 256);
-        hipLaunchKernelGGL(scatter_all, dim3(blocks), dim3(256), 0, c.stream, a);
+        const int blocks = a.bPT + a.bEE + a.bG + (int)blocks_for(capM, kCatThreads);
+        hipLaunchKernelGGL(scatter_all, dim3(blocks), dim3(kCatThreads), 0, c.stream, a);
         CIPC_CHECK_LAUNCH();
     }
     // PP/PE map: sort packed keys, run-length encode (std::map order with multiplicity); the

@@ -74,7 +74,7 @@ struct ActiveSetScratch {
     DBuf<int> candUPT, candUEE, candPT, candEE, ownPT, ownEE, catPT, catEE;
     DBuf<int4> recPT, recEE;
     DBuf<int2> auxEE;
-    DBuf<int4> pos_all;   // per-hit exclusive counts of four categories: point hits, then edge hits
+    DBuf<int4> cat_sums;   // category counts of every block of hits
     DBuf<unsigned long long> mkeys, mkeys_sorted, ukeys;
     DBuf<int> ucounts, nruns;
 };
