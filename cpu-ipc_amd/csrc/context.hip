@@ -950,6 +950,15 @@ void enqueue_iteration(cipc_gpu_context* c, double kappa, bool energy, const Ite
     if (t) CIPC_HIP(hipEventRecord(t->ev[0], c->stream));
     contact_records_prepare(*c);
     CIPC_HIP(hipEventRecord(c->it_start, c->stream));
+    // a batch goes as a graph, whose branches are started in this order: its full CCD is as long
+    // as the active set and starts beside it
+    const bool batch = c->sc.S > 1;
+    auto early = [&] {
+        CIPC_HIP(hipStreamWaitEvent(c->sbs, c->it_start, 0));
+        if (t) CIPC_HIP(hipEventRecord(t->s0, c->sbs));
+        step_bound_early(*c, c->sbs);
+    };
+    if (batch) early();
     compute_active_set(*c, false);   // contact_assemble publishes the counts
     if (t) CIPC_HIP(hipEventRecord(t->ev[1], c->stream));
     CIPC_HIP(hipEventRecord(c->as_done, c->stream));
@@ -960,10 +969,8 @@ void enqueue_iteration(cipc_gpu_context* c, double kappa, bool energy, const Ite
     friction_records_launch(*c, c->aux);
     CIPC_HIP(hipEventRecord(c->join, c->aux));
     contact_assemble(*c, kappa, true);
-    // the step bound after the barrier records: it has slack, the main stream has none
-    CIPC_HIP(hipStreamWaitEvent(c->sbs, c->it_start, 0));
-    if (t) CIPC_HIP(hipEventRecord(t->s0, c->sbs));
-    step_bound_early(*c, c->sbs);
+    // a scene's step bound after the barrier records: it has slack, the main stream has none
+    if (!batch) early();
     CIPC_HIP(hipStreamWaitEvent(c->sbs, c->as_done, 0));
     step_bound_partial(*c, c->sbs);
     if (t) CIPC_HIP(hipEventRecord(t->s1, c->sbs));
