@@ -25,6 +25,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <exception>
 
 namespace cipc {
 
@@ -1001,6 +1002,16 @@ void pcg_run(Context& c, const Layout& L, int S, const T* val, const Prec<T>& M,
     read_scalars(c, g.sc + (size_t)(it & 1) * S, S, h);
 }
 
+// Waits for the stream when a solve ends with an error: its iterations in flight still write the
+// pinned progress words, which the next solve clears from the host and must find its own.
+struct DrainOnError {
+    Context& c;
+    const int pending = std::uncaught_exceptions();
+    ~DrainOnError() {
+        if (std::uncaught_exceptions() > pending) (void)hipStreamSynchronize(c.stream);
+    }
+};
+
 // Per-scene state of the FP64 refinement.
 struct Refine {
     int iters = 0, outer = 0;
@@ -1059,6 +1070,7 @@ void linear_solve_scenes(Context& c, int precision, int preconditioner, double r
     Scene& s = c.sc;
     const int V = s.V, n = 3 * V, S = s.S;
     SolveBuffers& w = c.solve;
+    const DrainOnError drain{c};
     const Layout L = make_layout(c);
     const int ng = L.ng;
     w.part.resize((size_t)4 * ng);
