@@ -74,7 +74,9 @@ struct DBuf {
 // Grown-on-demand pinned host buffer: the destination of asynchronous device-to-host copies
 // that the host reads after a later synchronisation of the stream (so that one
 // synchronisation serves several results).  Grown only while no copy into it is pending.
-template <typename T>
+// Polled: words that kernels write while the host reads them, in coherent (fine-grained) memory,
+// which the default is only where the environment leaves it so.
+template <typename T, bool Polled = false>
 struct PinnedBuf {
     T* p = nullptr;
     size_t cap = 0;
@@ -90,7 +92,7 @@ struct PinnedBuf {
         if (p) CIPC_HIP(hipHostFree(p));
         p = nullptr;
         cap = 0;
-        CIPC_HIP(hipHostMalloc(reinterpret_cast<void**>(&p), want * sizeof(T), hipHostMallocDefault));
+        CIPC_HIP(hipHostMalloc(reinterpret_cast<void**>(&p), want * sizeof(T), Polled ? hipHostMallocCoherent : hipHostMallocDefault));
         cap = want;
     }
 };

@@ -238,7 +238,7 @@ struct Context {
     hipEvent_t read_ev[kReadSlots] = {};
     PinnedBuf<unsigned long long> pin_slots;
     PinnedBuf<double> pin_energy;
-    PinnedBuf<int> pin_pcg;            // a solve's progress, written by its kernels
+    PinnedBuf<int, true> pin_pcg;      // a solve's progress, written by its kernels
     bool assembled = false;    // a system exists for the linear solve
     SolveBuffers solve;
     int collisions = 0;

@@ -23,6 +23,9 @@ static int solve_fails(int preconditioner, int precision, int at) {
     EXPECT(failed);
     EXPECT(fake::launches > at);
     EXPECT(fake::in_flight == 0);
+    // the host polls the progress words while the kernels run: memory that is coherent whatever the
+    // environment's default is
+    if (c.pin_pcg.p) EXPECT(fake::pinned.at(c.pin_pcg.p) & hipHostMallocCoherent);
     return 0;
 }
 
