@@ -65,12 +65,12 @@ namespace cipc {
 // 381 on two 11^3.
 constexpr size_t kReadChunkMin = 256 << 10, kReadChunkMax = 1 << 20;
 void read_arrays_prepare(Context& c, size_t largest) {
-    if (c.read_chunk > 0 && c.read_chunk >= std::min(largest, kReadChunkMax)) return;
-    c.read_chunk = std::min(std::max((largest + 4095) / 4096 * 4096, kReadChunkMin), kReadChunkMax);
-    c.pin_arrays.reserve(kReadSlots * c.read_chunk);
+    if (c.pin_arrays.cap > 0 && c.pin_arrays.cap / kReadSlots >= std::min(largest, kReadChunkMax)) return;
+    c.pin_arrays.reserve(kReadSlots * std::min(std::max((largest + 4095) / 4096 * 4096, kReadChunkMin), kReadChunkMax));
 }
 void read_arrays(Context& c, std::initializer_list<HostArray> arrays) {
-    if (c.read_chunk == 0) read_arrays_prepare(c, kReadChunkMin);
+    if (c.pin_arrays.cap == 0) read_arrays_prepare(c, kReadChunkMin);
+    const size_t chunk = c.pin_arrays.cap / kReadSlots;   // a slot: what could be allocated
     struct Piece {
         char* host;
         const char* dev;
@@ -83,8 +83,8 @@ void read_arrays(Context& c, std::initializer_list<HostArray> arrays) {
     for (const HostArray& a : arrays) {
         if (!a.host) continue;
         for (size_t off = 0; off < a.bytes;) {
-            if (used >= c.read_chunk) { ++slot; used = 0; }
-            const size_t n = std::min(a.bytes - off, c.read_chunk - used);
+            if (used >= chunk) { ++slot; used = 0; }
+            const size_t n = std::min(a.bytes - off, chunk - used);
             pieces.push_back({static_cast<char*>(a.host) + off, static_cast<const char*>(a.dev) + off, n, used, slot});
             used += (n + 63) / 64 * 64;
             off += n;
@@ -92,7 +92,7 @@ void read_arrays(Context& c, std::initializer_list<HostArray> arrays) {
     }
     const int slots = pieces.empty() ? 0 : slot + 1;
     size_t issued = 0, moved = 0;
-    auto where = [&](const Piece& p) { return c.pin_arrays.p + (size_t)(p.slot % kReadSlots) * c.read_chunk + p.at; };
+    auto where = [&](const Piece& p) { return c.pin_arrays.p + (size_t)(p.slot % kReadSlots) * chunk + p.at; };
     auto issue = [&](int k) {
         for (; issued < pieces.size() && pieces[issued].slot == k; ++issued)
             CIPC_HIP(hipMemcpyAsync(where(pieces[issued]), pieces[issued].dev, pieces[issued].bytes, hipMemcpyDeviceToHost, c.stream));

@@ -232,9 +232,8 @@ struct Context {
     PinnedBuf<int> pin_nnz;
     PinnedBuf<int> pin_as;     // counts of the active-set construction
     PinnedBuf<unsigned char> pin_rb;   // staging of read_back
-    // staging of read_arrays: kReadSlots slots of read_chunk bytes, an event for each
+    // staging of read_arrays: kReadSlots slots in equal parts, an event for each
     PinnedBuf<unsigned char> pin_arrays;
-    size_t read_chunk = 0;
     hipEvent_t read_ev[kReadSlots] = {};
     PinnedBuf<unsigned long long> pin_slots;
     PinnedBuf<double> pin_energy;

@@ -39,6 +39,8 @@ hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t)
 hipError_t hipGetLastError() { const hipError_t e = fake::last; fake::last = hipSuccess; return e; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { std::memcpy(d, s, n); return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { fake::in_flight = 0; return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamQuery(hipStream_t) { return fake::in_flight ? hipErrorNotReady : hipSuccess; }
 }
 

@@ -11,7 +11,7 @@ HERE = os.path.join(ROOT, "tests", "host_failures")
 PKG = os.path.join(ROOT, "cpu-ipc_amd")
 
 
-@pytest.mark.parametrize("program", ["solve"])
+@pytest.mark.parametrize("program", ["solve", "read_arrays"])
 def test_failure(program, tmp_path):
     exe = str(tmp_path / program)
     r = subprocess.run(["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-host-only", "-O1", "-std=c++17", "-Wno-unused-result",
