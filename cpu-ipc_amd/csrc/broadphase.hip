@@ -667,7 +667,12 @@ __device__ inline void ee_classify(int u, const int* __restrict__ dc, int Es, co
 // its own block, and ballots within a block.  Only the hits there are, not the capacity, are
 // read, and no position is stored: a device-wide scan over the capacities wrote 16 bytes a
 // slot (with the scatter 333 us on a batch of 40 scenes and 55 on a folded 128^2 cloth, now 110 and 19).
-constexpr int kCatBlock = 1024, kCatThreads = 256;
+// What the work-groups read grows with the square of the blocks, so where the capacities hold
+// more than kOwnCounts blocks one work-group adds the counts up once (category_starts).  The
+// line lies where a launch costs what the sums do: folded cloths with 920 blocks of hits take 15.6 us
+// adding up themselves and 10.8 + 5.0 with the launch, 2,450 blocks 26.5 and 19.5 + 7.0, 12,900 blocks
+// 326 and 117 + 23.
+constexpr int kCatBlock = 1024, kCatThreads = 256, kOwnCounts = 2048, kStartThreads = 1024;
 // Category masks of the point-triangle hits and of the edge-edge hits.
 __device__ constexpr unsigned kCatPT[4] = {1u << kSelfPT, 1u << kMap, (1u << kNone) | (1u << kSelfPT) | (1u << kMap), 0u};
 __device__ constexpr unsigned kCatEE[4] = {1u << kSelfEE, 1u << kMap, (1u << kMolPE) | (1u << kMolEE),
@@ -712,6 +717,44 @@ __global__ __launch_bounds__(kCatThreads) void category_counts(const int* __rest
     if ((threadIdx.x & 63) == 0) sh[w] = t;
     __syncthreads();
     if (threadIdx.x == 0) sums[blockIdx.x] = add4(add4(sh[0], sh[1]), add4(sh[2], sh[3]));
+}
+// Every block's counts become the counts of the blocks of its kind before it; the totals of both
+// kinds follow at sums[bPT + bEE].  One work-group.
+__global__ __launch_bounds__(kStartThreads) void category_starts(const int* __restrict__ dc, int bPT, int bEE, int4* __restrict__ sums) {
+    __shared__ int4 part[kStartThreads / 64], total;
+    if (dc[kDcFlags]) return;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int kind = 0; kind < 2; ++kind) {
+        int4* s = sums + (kind ? bPT : 0);
+        const int n = (dc[kind ? kDcEE : kDcPT] + kCatBlock - 1) / kCatBlock;
+        int4 base = make_int4(0, 0, 0, 0);
+        for (int b0 = 0; b0 < n; b0 += kStartThreads) {
+            const int b = b0 + threadIdx.x;
+            const int4 v = b < n ? s[b] : make_int4(0, 0, 0, 0);
+            int4 x = v;   // inclusive over the wavefront
+            for (int d = 1; d < 64; d <<= 1) {
+                const int4 y = make_int4(__shfl_up(x.x, d), __shfl_up(x.y, d), __shfl_up(x.z, d), __shfl_up(x.w, d));
+                if (lane >= d) x = add4(x, y);
+            }
+            if (lane == 63) part[w] = x;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                int4 t = make_int4(0, 0, 0, 0);
+                for (int k = 0; k < kStartThreads / 64; ++k) {
+                    const int4 p = part[k];
+                    part[k] = t;
+                    t = add4(t, p);
+                }
+                total = t;
+            }
+            __syncthreads();
+            const int4 at = add4(base, part[w]);
+            if (b < n) s[b] = make_int4(at.x + x.x - v.x, at.y + x.y - v.y, at.z + x.z - v.z, at.w + x.w - v.w);
+            base = add4(base, total);
+            __syncthreads();   // part and total are the next round's
+        }
+        if (threadIdx.x == 0) sums[bPT + bEE + kind] = base;
+    }
 }
 // PP/PE map key: (c0 + V, c1, c2 + 1) packed with `bits` per field preserves the signed
 // lexicographic order of std::map<EncodedContact, int> (all keys have c3 = -1).
@@ -779,12 +822,12 @@ __device__ inline void ground_scatter(int s, int Vs, const int* __restrict__ sv,
 }
 // In one launch (the four parts write disjoint entries): work-groups [0, bPT) place the point
 // hits, the next bEE the edge hits, the next bG the ground entries, the rest write the map keys'
-// all-ones tail.  Every work-group with work adds up the blocks' counts; the first publishes the
-// totals (category_totals).  Nothing is placed when a capacity was exceeded: the host builds the
+// all-ones tail.  Every work-group with work adds up the blocks' counts (or, with own_counts 0,
+// reads what category_starts made of them); the first publishes the totals (category_totals).  Nothing is placed when a capacity was exceeded: the host builds the
 // set again.
 struct ScatterArgs {
     int* dc;
-    int V, bits, Vs, capM, bPT, bEE, bG;
+    int V, bits, Vs, capM, bPT, bEE, bG, own_counts;
     const int *catPT, *ownPT, *candPT, *catEE, *ownEE, *candEE, *sv, *fg, *pg;
     const int4 *sums, *recPT, *recEE;
     const int2* auxEE;
@@ -823,7 +866,11 @@ __global__ __launch_bounds__(kCatThreads) void scatter_all(ScatterArgs a) {
     if (!first && ((pt && b * kCatBlock >= nPT) || (ee && (b - a.bPT) * kCatBlock >= nEE))) return;
     // the totals of both kinds (ta, tb), and the counts before this block (of its kind)
     int4 ta = make_int4(0, 0, 0, 0), tb = ta, at = ta;
-    {
+    if (!a.own_counts) {
+        ta = a.sums[a.bPT + a.bEE];
+        tb = a.sums[a.bPT + a.bEE + 1];
+        if ((pt && b * kCatBlock < nPT) || ee) at = a.sums[b];
+    } else {
         const int4 zero = ta;
         const int kPT = (nPT + kCatBlock - 1) / kCatBlock, kEE = (nEE + kCatBlock - 1) / kCatBlock;
         for (int k = threadIdx.x; k < kPT + kEE; k += kCatThreads) {
@@ -1100,9 +1147,12 @@ void compute_active_set(Context& c, bool publish) {
     CIPC_CHECK_LAUNCH();
     // category counts of every block of hits
     const int blocksPT = (int)blocks_for(capPT, kCatBlock), blocksEE = (int)blocks_for(capEE, kCatBlock);
-    b.cat_sums.resize((size_t)blocksPT + blocksEE);
+    b.cat_sums.resize((size_t)blocksPT + blocksEE + 2);   // then the totals
     hipLaunchKernelGGL(category_counts, dim3(blocksPT + blocksEE), dim3(kCatThreads), 0, c.stream, dc, blocksPT, b.catPT.p, b.catEE.p,
                        b.cat_sums.p);
+    const bool own_counts = blocksPT + blocksEE <= kOwnCounts;
+    if (!own_counts)
+        hipLaunchKernelGGL(category_starts, dim3(1), dim3(kStartThreads), 0, c.stream, dc, blocksPT, blocksEE, b.cat_sums.p);
     CIPC_CHECK_LAUNCH();
     // PP/PE map keys need the vertex count to fit three fields in 64 bits
     int bits = 1;
@@ -1115,7 +1165,7 @@ void compute_active_set(Context& c, bool publish) {
     {
         ScatterArgs a;
         a.dc = dc; a.V = s.V; a.bits = bits; a.Vs = Vs; a.capM = capM;
-        a.bPT = blocksPT; a.bEE = blocksEE; a.bG = (int)blocks_for(Vs, kCatThreads); a.sums = b.cat_sums.p;
+        a.bPT = blocksPT; a.bEE = blocksEE; a.bG = (int)blocks_for(Vs, kCatThreads); a.own_counts = own_counts; a.sums = b.cat_sums.p;
         a.catPT = b.catPT.p; a.ownPT = b.ownPT.p; a.candPT = b.candPT.p; a.recPT = b.recPT.p;
         a.catEE = b.catEE.p; a.ownEE = b.ownEE.p; a.candEE = b.candEE.p; a.recEE = b.recEE.p; a.auxEE = b.auxEE.p;
         a.sv = s.sv.p; a.fg = cG; a.pg = oG; a.self_set = c.self_set.p; a.ee_set = c.ee_set.p; a.ee_ie = c.ee_ie.p;
