@@ -47,6 +47,7 @@ EXPORTS = (
     "cipc_gpu_eval_snh", "cipc_gpu_eval_cloth", "cipc_gpu_eval_hinge", "cipc_gpu_eval_distance", "cipc_gpu_eval_make_pd", "cipc_gpu_eval_contact_pd",
     "cipc_gpu_eval_accd",
     "cipc_gpu_eval_classify",
+    "cipc_gpu_eval_walk",
 )
 
 
@@ -192,6 +193,7 @@ def load(path: str = LIB_PATH):
         "cipc_gpu_eval_contact_pd": [C.c_int, C.c_int, _dp, _dp],
         "cipc_gpu_eval_accd": [C.c_int, C.c_int, _dp, _dp, C.c_double, C.c_double, _dp],
         "cipc_gpu_eval_classify": [C.c_int, C.c_int, _dp, _ip],
+        "cipc_gpu_eval_walk": [C.c_int, _dp, C.c_int, _dp, C.c_double, C.c_int, C.c_int, C.c_int, _ip, _ip],
     }
     for name, args in sig.items():
         fn = getattr(L, name)
@@ -719,3 +721,18 @@ def eval_classify(kind, pts):
     out = np.zeros(n, np.int32)
     _check(load().cipc_gpu_eval_classify(n, kind, _dptr(pts), _iptr(out)))
     return out
+
+
+def eval_walk(boxes, queries=None, gap=0.0, bits=0, depth=64, max_hits=None):
+    """The hits of each query's walk over a tree of boxes (n, 6), a list of arrays: with queries
+    (nq, 6) the boxes that may come within gap, else the overlapping boxes of later leaves, each once
+    or more."""
+    boxes = _d(np.asarray(boxes).reshape(-1, 6))
+    q = None if queries is None else _d(np.asarray(queries).reshape(-1, 6))
+    n = boxes.shape[0]
+    nq = n if q is None else q.shape[0]
+    max_hits = max_hits or 2 * n
+    counts, hits = np.zeros(nq, np.int32), np.zeros((nq, max_hits), np.int32)
+    _check(load().cipc_gpu_eval_walk(n, _dptr(boxes), nq, None if q is None else _dptr(q), gap, bits, depth, max_hits, _iptr(counts),
+                                     _iptr(hits)))
+    return [hits[k, :min(c, max_hits)] for k, c in enumerate(counts)]

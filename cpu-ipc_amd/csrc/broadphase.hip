@@ -1351,6 +1351,54 @@ void scene_intersections(Context& c, int* out) {
     for (int k = 0; k < S; ++k) out[k] = (h[k] != 0 || h[S + k] != 0) ? 1 : 0;
 }
 
+// ---------------------------------------------------------------------------------
+// Evaluation entry point (tests): the walks over boxes of the caller's
+// ---------------------------------------------------------------------------------
+// queries: all leaves a query may overlap, in any order (query_hits); null: each box's own query
+// for the leaves after its own, the overlapping pairs once or more (pair_walk)
+__global__ __launch_bounds__(64) void walk_eval_kernel(TreeView t, const Box* __restrict__ box, int nq, const Box* __restrict__ queries,
+                                                       double gap, int bits, int depth, int max_hits, int* __restrict__ counts,
+                                                       int* __restrict__ hits) {
+    __shared__ int lds[kWalkInts];
+    __shared__ int2 met[kPairQueue], kept[kPairQueue];
+    const WalkGroup G(bits, depth);
+    const int i = (blockIdx.x << (4 - bits)) + G.g, q = i < nq ? i : -1;
+    if (queries) {
+        const int n = query_hits(t, G, q >= 0, q >= 0 ? queries[q] : Box{}, gap, -1, lds, [&](int k, int prim) {
+            if (k < max_hits) hits[(size_t)q * max_hits + k] = prim;
+        });
+        if (q >= 0 && G.l == 0) counts[q] = n;
+        return;
+    }
+    pair_walk<true>(t, G, q, q >= 0 ? box[q] : Box{}, q >= 0 ? t.leafpos[q] : 0, lds, met, kept,
+                    [&](int2 pr) { return overlaps(box[pr.x], box[pr.y], 0.0); },
+                    [&](bool on, int2 pr) {
+                        if (!on) return;
+                        const int k = atomicAdd(counts + pr.x, 1);
+                        if (k < max_hits) hits[(size_t)pr.x * max_hits + k] = pr.y;
+                    });
+}
+void eval_walk(int n, const double* boxes, int nq, const double* queries, double gap, int bits, int depth, int max_hits, int* counts,
+               int* hits) {
+    Context c;
+    LBVH t;
+    DBuf<Box> q;
+    DBuf<int> dc, dh;
+    t.prim.resize(n); dc.resize(nq); dh.resize((size_t)nq * max_hits);
+    CIPC_HIP(hipMemcpy(t.prim.p, boxes, sizeof(Box) * n, hipMemcpyHostToDevice));
+    if (queries) {
+        q.resize(nq);
+        CIPC_HIP(hipMemcpy(q.p, queries, sizeof(Box) * nq, hipMemcpyHostToDevice));
+    }
+    hipLaunchKernelGGL(zero_int, dim3(blocks_for(nq, 256)), dim3(256), 0, c.stream, dc.p, nq);
+    build_tree(c, t, n);
+    hipLaunchKernelGGL(walk_eval_kernel, dim3(blocks_for((size_t)nq << bits, 16)), dim3(64), 0, c.stream,
+                       TreeView{t.n, t.nodes.p, t.wide.p, t.leafpos.p}, t.prim.p, nq, q.p, gap, bits, depth, max_hits, dc.p, dh.p);
+    CIPC_CHECK_LAUNCH();
+    CIPC_HIP(hipMemcpy(counts, dc.p, sizeof(int) * nq, hipMemcpyDeviceToHost));
+    CIPC_HIP(hipMemcpy(hits, dh.p, sizeof(int) * nq * (size_t)max_hits, hipMemcpyDeviceToHost));
+}
+
 bool any_intersection(Context& c) {
     std::vector<int> r(c.sc.S);
     scene_intersections(c, r.data());

@@ -1413,6 +1413,15 @@ int cipc_gpu_eval_classify(int n, int kind, const double* pts, int* type) {
         if (n) cipc_gpu_eval_classify_impl(n, kind, pts, type);
     });
 }
+int cipc_gpu_eval_walk(int n, const double* boxes, int nq, const double* queries, double gap, int bits, int depth, int max_hits,
+                       int* counts, int* hits) {
+    return guard([&] {
+        require(n > 0 && n <= 1 << 24 && boxes && counts && hits, "invalid boxes or null output");
+        require(nq > 0 && nq <= 1 << 24 && (queries || nq == n) && max_hits > 0, "invalid queries");
+        require(bits >= 0 && bits <= 4 && depth >= 1 && depth <= 64, "bits is 0..4, depth 1..64");
+        eval_walk(n, boxes, nq, queries, gap, bits, depth, max_hits, counts, hits);
+    });
+}
 
 }  // extern "C"
 

@@ -302,6 +302,8 @@ void publish_nnz(Context& c, hipStream_t st);
 void exclusive_scan_int(Context& c, const int* in, int* out, int n);
 // broadphase.hip
 void build_tree(Context& c, LBVH& t, int n);
+void eval_walk(int n, const double* boxes, int nq, const double* queries, double gap, int bits, int depth, int max_hits, int* counts,
+               int* hits);
 void build_static_trees(Context& c);
 // on stream st (the step bound may run beside the assembly); temporary storage of its own
 void build_swept_trees(Context& c, const unsigned long long* abits, hipStream_t st);

@@ -60,17 +60,20 @@ __device__ inline bool overlaps_f(const WalkBox& q, const float* lo, const float
 // is walked again over the exact boxes by its first lane (depth first along the skip pointers,
 // CPULinearBVH::query semantics, LBVH.cpp:252-282, without the final sort), after the others:
 // exact() is true for its group from then on, and what it met before is met again.
-constexpr int kWalkInts = 1024;   // stack entries of a wavefront, 64 << bits of each query
+constexpr int kWalkInts = 1024;   // stack entries of a wavefront, kWalkDepth << bits of each query
+constexpr int kWalkDepth = 64;
 // order of the wavefront's own LDS accesses (they execute in issue order)
 __device__ inline void walk_order() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-// a query's lanes in the wavefront
+// a query's lanes in the wavefront; fewer entries than there is room for only where the evaluation
+// entry point asks for them, to make walks run out
 struct WalkGroup {
-    int bits, g, l;   // group, lane in the group
-    __device__ explicit WalkGroup(int b) : bits(b), g((threadIdx.x & 63) >> (b + 2)), l(threadIdx.x & ((4 << b) - 1)) {}
+    int bits, g, l, cap;   // group, lane in the group, stack entries of a query
+    __device__ explicit WalkGroup(int b, int depth = kWalkDepth)
+        : bits(b), g((threadIdx.x & 63) >> (b + 2)), l(threadIdx.x & ((4 << b) - 1)), cap(depth << b) {}
     // the group's part of a ballot, and how many of its bits come before this lane
     __device__ unsigned long long part(unsigned long long m) const {
         const int lanes = 4 << bits;
@@ -98,7 +101,7 @@ class GroupWalk {
 
 public:
     __device__ GroupWalk(const TreeView& t_, const WalkGroup& G_, bool active, const Box& q_, double gap_, int after_, int* lds)
-        : t(t_), G(G_), q(q_), gap(gap_), after(after_), stk(lds + G_.g * (64 << G_.bits)), w(walk_box(q_, gap_)), sp(0), left(t_.n),
+        : t(t_), G(G_), q(q_), gap(gap_), after(after_), stk(lds + G_.g * (kWalkDepth << G_.bits)), w(walk_box(q_, gap_)), sp(0), left(t_.n),
           bin(-1), over(false) {
         if (active && t.n > 1) {
             if (G.l == 0) stk[0] = 0;
@@ -115,7 +118,7 @@ public:
         bool yes = false;
         int prim = 0;
         if (__any(sp > 0)) {
-            const int slot = G.l >> 2, k = G.l & 3, cap = 64 << G.bits;
+            const int slot = G.l >> 2, k = G.l & 3;
             const int n = min(sp, 1 << G.bits);
             const bool on = slot < n;
             const int node = on ? stk[sp - 1 - slot] : 0;
@@ -133,7 +136,7 @@ public:
             const bool in = ov && c.child >= 0;
             const unsigned long long m = G.part(__ballot(in));
             const int add = __popcll(m);
-            if (sp + add > cap || (--left <= 0 && sp + add > 0)) {
+            if (sp + add > G.cap || (--left <= 0 && sp + add > 0)) {
                 restart();
             } else {
                 if (in) stk[sp + G.before(m)] = c.child;

@@ -444,6 +444,15 @@ int cipc_gpu_eval_make_pd(int n, int dim, double* H);
 int cipc_gpu_eval_contact_pd(int n, int nverts, double* H, const double* G);
 int cipc_gpu_eval_accd(int n, int kind, const double* pts, const double* dirs, double eta, double thickness, double* toc);
 int cipc_gpu_eval_classify(int n, int kind, const double* pts, int* type);
+/*  walk:     a tree over n boxes (lower, upper: 6n), walked by 4 * 2^bits lanes per query with a
+ *            stack of depth * 2^bits records (64 in the library's own walks; a query that runs
+ *            out is walked again over the exact boxes).  counts (nq) and the first max_hits of
+ *            each query's hits (nq * max_hits, in any order): with queries (6nq) the boxes that may
+ *            come within gap of each (a superset of those that do), without (nq = n) the boxes
+ *            that overlap box q and whose leaf follows its own, each once or more
+ *            (LBVH.cpp:252-282) */
+int cipc_gpu_eval_walk(int n, const double* boxes, int nq, const double* queries, double gap, int bits, int depth, int max_hits,
+                       int* counts, int* hits);
 
 #ifdef __cplusplus
 }
