@@ -17,6 +17,13 @@ def test_more_than_one_gpu_is_refused():
     assert "one GPU" in r.stderr or "single" in r.stderr
 
 
+def test_lanes_of_the_tuned_walks():
+    sys.path.insert(0, ROOT)
+    import bench
+    # candidate c of a walk runs 4 * 2^c lanes per query (cipc_gpu.h)
+    assert bench.lanes_per_query({"full_ccd_pt": (0, [0.1] * 5), "active_ee": (4, [0.1] * 5)}) == {"full_ccd_pt": 4, "active_ee": 64}
+
+
 def test_elastic_algorithmic_bytes():
     sys.path.insert(0, ROOT)
     import bench
