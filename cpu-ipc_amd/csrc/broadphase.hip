@@ -16,7 +16,7 @@
 // results do not depend on the topology, so it is rebuilt only every kMaxRefits fits.
 //
 // Active set: each surface vertex (point-triangle) and surface edge (edge-edge) query walks the
-// tree with a group of lanes (group_walk) that buffers its first candidates; a second pass
+// tree with a group of lanes (GroupWalk) that buffers its first candidates; a second pass
 // packs them (walking again only where they did not fit); one thread per candidate places it by
 // its primitive id, as the reference's query sorts them, and classifies it.
 // Compaction reproduces the reference's serial order: partial-CCD pairs, then Self_ActiveSet =
@@ -1284,7 +1284,7 @@ __device__ inline bool seg_tri(d3 e0, d3 e1, d3 t0, d3 t1, d3 t2) {
     return xs[0] >= 0.0 && xs[1] >= 0.0 && xs[0] + xs[1] <= 1.0 && xs[2] >= 0.0 && xs[2] <= 1.0;
 }
 // hit[0] (one scene) or hit[scene] (batch) is set for a face that an edge crosses.  The edges
-// walk the face tree (group_walk), a group of lanes each; the pairs whose boxes may overlap are
+// walk the face tree (GroupWalk), a group of lanes each; the pairs whose boxes may overlap are
 // queued in LDS and tested 64 at a time, so that the test's lanes are full whatever query found
 // them.  One lane per face, walking the binary tree of the edges and testing on the way, took 162 us
 // on four 20^3 cubes; this takes 27, and the edge tree needs no refit.

