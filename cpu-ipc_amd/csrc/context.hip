@@ -1028,7 +1028,7 @@ void drop_graph(cipc_gpu_context* c) {
 // while capturing, or the capture failed).  t0/t1 bracket the launch.
 bool iteration_graph(cipc_gpu_context* c, double kappa, bool energy, hipEvent_t t0, hipEvent_t t1) {
     // by default a batch goes as one graph launch and a single scene eagerly (measured no
-    // faster as a graph: launching the graph's ~120 nodes costs the host what the launches do)
+    // faster as a graph: launching the graph's nodes costs the host what the launches do)
     const bool on = c->graph.mode < 0 ? c->sc.S > 1 : c->graph.mode == 1;
     // (an enqueue that was cut short has left the bucket counts for an eager one to clear)
     if (!on || !trees_refit_only(c) || c->capS == 0 || c->as.capPT == 0 || c->bucket_cnt_clear == 0) return false;
